@@ -253,6 +253,9 @@ size_t mm_work_bytes(int in_dim, int out_dim, int batch) {
     if (bp >= batch) break;
   }
   if (in_dim % 1024 == 0) n = std::max(n, kq::mmw_workspace_bytes(in_dim, out_dim, std::min(batch, 64)));
+  // From 64 vectors on, room for any batch, so that a stream warmed up with 64
+  // may capture larger products.
+  n = std::max(n, kq::gemm_workspace_bytes(in_dim, out_dim, batch >= 64 ? kq::GEMM_STEP : batch));
   return n;
 }
 
@@ -268,7 +271,8 @@ struct MvWorkspace {
     if (part.ensure(std::max<size_t>(pf, 64), "hipMalloc partials")) return -1;
     if (batch > 1 && mm.ensure(mm_work_bytes(in_dim, out_dim, batch), "hipMalloc mfma")) return -1;
     bool grew = false;
-    if (count.ensure(kq::packed_counters(out_dim), "hipMalloc counters", &grew)) return -1;
+    const size_t nc = kq::packed_counters(out_dim);
+    if (count.ensure(batch > 1 ? std::max(nc, kq::GEMM_COUNTERS) : nc, "hipMalloc counters", &grew)) return -1;
     return grew ? check(hipMemset(count.p, 0, count.n * sizeof(unsigned)), "hipMemset counters") : 0;
   }
 };
@@ -278,7 +282,9 @@ struct MvWorkspace {
 // 2 the 64-vector and 3 the 16-vector MFMA kernel, 4 the one-pass kernel
 // (kq_mmv.hip), 5 the batch-1 kernel for up to 4 vectors per launch and 6
 // the wave-per-column kernel (kq_mmw.hip), where the kind has one.
-// The pick for Q4_K and Q6_K (measured on MI355X at 4096x4096 and
+// The pick is the many-vector kernel (kq_gemm.hip) where gemm_takes says so:
+// every kind above 64 vectors, and most batches above 4 to 16 on all but the
+// smallest matrices.  Below its line, for Q4_K and Q6_K (measured on MI355X at 4096x4096 and
 // 14336x4096, `small_batch` of bench.py):
 //   up to 4 vectors: the batch-1 kernel on 4 vectors where its batch-1
 //     plan is 16-row workgroups (and Q6_K at 2 vectors), else one pass;
@@ -307,7 +313,8 @@ thread_local int g_mm_engine = 0;
 
 // The kernel family of a batched product and how many vectors each launch
 // takes: 0 the multi-vector VALU kernel, 1 the 16-vector and 2 the 64-vector
-// MFMA kernel.
+// MFMA kernel, 3 the one-pass, 4 the batch-1, 5 the wave-per-column and 6 the
+// many-vector kernel.
 struct MmRoute {
   int family, step;
 };
@@ -325,6 +332,7 @@ MmRoute mm_route(int kind, int in_dim, int out_dim, int batch) {
   // Q6_K in launches of at most 32 vectors: the 64-vector kernel's Q6_K
   // variant runs out of registers above 32 (14336x4096: 359 us for 64
   // vectors in one launch, 82 us per 32).
+  if (eng == 0 && kq::gemm_takes(kind, in_dim, out_dim, batch)) return {6, kq::GEMM_STEP};
   if (eng == 4 && kq::mmv_kind(kind)) return {3, 64};
   if (eng == 5 && kq::matvec_nv_takes(kind, in_dim, out_dim)) return {4, 4};
   if (eng == 6 && kq::mmw_takes(kind, in_dim)) return {5, 64};
@@ -356,6 +364,11 @@ MmRoute mm_route(int kind, int in_dim, int out_dim, int batch) {
 size_t mm_launch_need(int kind, int in_dim, int out_dim, int batch) {
   if (batch <= 1) return 0;
   const MmRoute r = mm_route(kind, in_dim, out_dim, batch);
+  if (r.family == 6) {
+    size_t n = kq::gemm_launch_bytes(in_dim, out_dim, std::min(batch, r.step));
+    if (batch > r.step && batch % r.step) n = std::max(n, kq::gemm_launch_bytes(in_dim, out_dim, batch % r.step));
+    return n;
+  }
   if (r.family == 5) return kq::mmw_workspace_bytes(in_dim, out_dim, std::min(batch, r.step));
   if (r.family == 0 || r.family >= 3) return 0;
   if (r.family == 1) return kq::mm16_workspace_bytes(in_dim, out_dim);
@@ -378,6 +391,8 @@ hipError_t matmul_packed(int kind, const void* P, int in_dim, int out_dim, int b
       e = kq::launch_matvec_mfma_nv(kind, P, in_dim, out_dim, nb, xb, yb, st);
     else if (r.family == 3)
       e = kq::launch_matmul_mmv(kind, P, in_dim, out_dim, nb, xb, yb, st);
+    else if (r.family == 6)
+      e = kq::launch_gemm(kind, P, in_dim, out_dim, nb, xb, yb, ws.mm.p, ws.count.p, st);
     else if (r.family == 5)
       e = kq::launch_matmul_mmw(kind, P, in_dim, out_dim, nb, xb, yb, ws.mm.p, ws.count.p, st);
     else if (r.family == 1)

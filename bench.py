@@ -398,13 +398,41 @@ def small_batch_table(torch, aa, synth, seed, stream, engine=0):
     return table
 
 
+def gemm_takes(aa, kind, inp, out, B):
+    """gemm_takes of kq_gemm.hip for Q4_K and Q6_K: where the many-vector
+    kernel is the library's default pick."""
+    nsb, tiles = inp // 256, -(-out // 64)
+    units, narrow = nsb * tiles, tiles < 192
+    if B > 64:
+        return True
+    if kind == aa.Q4_K:
+        if B > 32:
+            return nsb >= 16
+        if B > 16:
+            return nsb >= 32 or units >= 3584
+        return B > 4 and narrow and (units >= (2048 if B > 8 else 3584) or nsb >= 48)
+    if B > 32:
+        return B > 48 or units > 1024 or nsb < 32
+    if B > 16:
+        return nsb >= 16
+    split16 = narrow and tiles >= 128 and nsb >= 16
+    if B > 8:
+        return units >= 3584 or nsb >= 48 or split16 or (B > 12 and nsb >= 16)
+    if B > 4:
+        return units >= 7168 or nsb >= 48 or split16
+    return B > 2 and units >= 16384
+
+
 def small_batch_kernel(aa, kind, inp, out, B):
     """The kernel the library's default small-batch pick runs (mm_route in
-    aspidagpu.hip) for Q4_K and Q6_K: up to 4 vectors the batch-1 kernel on
-    4 vectors where the batch-1 plan is 16-row workgroups (and Q6_K at 2),
-    else the one-pass kernel; the one-pass kernel up to 16 vectors and for
-    Q6_K above (the wave-per-column kernel above 32 vectors on at most 1024
-    (tile, column) pairs); Q4_K above 16 on the 64-vector MFMA kernel."""
+    aspidagpu.hip) for Q4_K and Q6_K: the many-vector kernel where gemm_takes
+    says so; else up to 4 vectors the batch-1 kernel on 4 vectors where the
+    batch-1 plan is 16-row workgroups (and Q6_K at 2), else the one-pass
+    kernel; the one-pass kernel up to 16 vectors and for Q6_K above (the
+    wave-per-column kernel above 32 vectors on at most 1024 (tile, column)
+    pairs); Q4_K above 16 on the 64-vector MFMA kernel."""
+    if gemm_takes(aa, kind, inp, out, B):
+        return "kq_gemm"
     units = (-(-out // 64)) * (inp // 256)
     tall = units >= 8192
     if kind == aa.Q6_K and B > 32 and units <= 1024 and inp % 1024 == 0:

@@ -150,13 +150,14 @@ int aspida_kq_matvec2_packed_dev(int kind_a, const void *packed_a, int out_a, fl
                                  const void *packed_b, int out_b, float *y_b, int in_dim, const float *x,
                                  void *stream);
 
-/* Y[batch][out_dim] = X[batch][in_dim] W^T for packed W: the small-batch
- * path.  Small batches run on a multi-vector VALU kernel, each row
- * bit-identical to aspida_kq_matvec_packed_dev on it: up to 4 rows for Q4_K
- * and Q6_K, whose larger batches run on MFMA (activations split into f16
- * hi + lo, exact integer codes, f32 scales; 64 rows per launch), and 8 rows
- * per launch for the other kinds.
- * x must be 16-byte aligned; workspace as for aspida_kq_matvec_packed_dev.
+/* Y[batch][out_dim] = X[batch][in_dim] W^T for packed W: any batch.  Products
+ * run on MFMA (activations split into f16 hi + lo, exact integer codes, f32
+ * scales), up to 512 vectors per weight pass, except few vectors of Q5_K,
+ * Q3_K, Q2_K and Q8_0 (up to 4 to 7 by shape, 24 on the smallest matrices),
+ * which run on the vector kernel, each row bit-identical to
+ * aspida_kq_matvec_packed_dev on it under aspida_kq_set_mv_engine(1).
+ * x must be 16-byte aligned; workspace as for aspida_kq_matvec_packed_dev
+ * (sized by in_dim, out_dim and the batch; from 64 vectors on for any batch).
  * The same math as the reference's batched kernels (gpu/gpu_matvec.cu:234-382)
  * without its batch limit of 32. */
 int aspida_kq_matmul_packed_dev(int kind, const void *packed, int in_dim, int out_dim, int batch,
@@ -409,7 +410,8 @@ int aspida_kq_set_mv_engine(int engine);
 
 /* Engine of the packed small-batch product (batch > 1 in
  * aspida_kq_matmul_packed_dev and aspida_gpu_matmul): 0 = the built-in choice
- * (Q4_K and Q6_K: up to 4 vectors on the batch-1 matrix-core kernel where
+ * (the many-vector kernel wherever it measured ahead: every kind above 64
+ * vectors, most matrices above 4 to 16; below that line, Q4_K and Q6_K: up to 4 vectors on the batch-1 matrix-core kernel where
  * the batch-1 plan is 16-row workgroups, else the one-pass kernel -- Q6_K
  * keeps the batch-1 kernel at 2 vectors -- then the one-pass kernel up to
  * 16 vectors (on matrices of at least 8192 64-row-by-256-column blocks,
