@@ -45,7 +45,9 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 constexpr int GX_AUX = 32 * 1024;
 constexpr int GX_SUM = GX_AUX + 1024;
 constexpr int GX_COL = 36 * 1024;
-constexpr int GX_RING = 4;             // 64-element stages (8 KB per vector block) in LDS
+// 64-element stages (8 KB per vector block) in LDS: as many as leave room for
+// three workgroups per CU (NV = 1) or two (NV = 2).
+constexpr int gx_ring(int nv) { return nv == 1 ? 6 : 4; }
 constexpr int GX_STAGE = 8 * 1024;
 constexpr int GX_GROUP = 8;
 
@@ -313,84 +315,203 @@ template <class P> struct GxW<Q8_0, P> {
   __device__ __forceinline__ S scales() const { return {sc}; }
 };
 
+// ---- the activation split ------------------------------------------------------
+//
+// Thread u (0..7, consecutive lanes) of one vector's column at x (null: zeros):
+// elements 32 u .. 32 u + 31 into fragments 4 u .. 4 u + 3.  frag(f, h) is where
+// the vector's 16 bytes of fragment f, lane half h go, sums(i, h) those of min-
+// term fragment i, inv where 1 / S goes.
+template <int SUMS, class F, class G>
+__device__ __forceinline__ void gx_split(const float* x, int u, F&& frag, G&& sums, uint8_t* inv) {
+  float4 v[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    v[i] = x ? reinterpret_cast<const float4*>(x + 32 * u)[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+  float a = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) a = fmaxf(a, fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w))));
+#pragma unroll
+  for (int o = 1; o < 8; o <<= 1) a = fmaxf(a, __shfl_xor(a, o, 64));
+  // S = 2^(14 - e) with a < 2^e, at most 2^116; 1 for zero or non-finite columns.
+  int e = 0;
+  const bool scaled = a > 0.f && __builtin_isfinite(a);
+  if (scaled) (void)frexpf(a, &e);
+  const int ex = scaled ? min(14 - e, 116) : 0;
+  const float S = ldexpf(1.f, ex);
+  if (u == 0) *reinterpret_cast<float*>(inv) = ldexpf(1.f, -ex);
+  float part[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    float q[4];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      float4 x0 = v[4 * h + 2 * b], x1 = v[4 * h + 2 * b + 1];
+      x0.x *= S; x0.y *= S; x0.z *= S; x0.w *= S;
+      x1.x *= S; x1.y *= S; x1.z *= S; x1.w *= S;
+      const h8 hi = {(_Float16)x0.x, (_Float16)x0.z, (_Float16)x0.y, (_Float16)x0.w,
+                     (_Float16)x1.x, (_Float16)x1.z, (_Float16)x1.y, (_Float16)x1.w};
+      const h8 lo = {(_Float16)(x0.x - (float)hi[0]), (_Float16)(x0.z - (float)hi[1]), (_Float16)(x0.y - (float)hi[2]),
+                     (_Float16)(x0.w - (float)hi[3]), (_Float16)(x1.x - (float)hi[4]), (_Float16)(x1.z - (float)hi[5]),
+                     (_Float16)(x1.y - (float)hi[6]), (_Float16)(x1.w - (float)hi[7])};
+      *reinterpret_cast<h8*>(frag(4 * u + 2 * b, h)) = hi;
+      *reinterpret_cast<h8*>(frag(4 * u + 2 * b + 1, h)) = lo;
+      q[2 * b] = (x0.x + x0.y) + (x0.z + x0.w);
+      q[2 * b + 1] = (x1.x + x1.y) + (x1.z + x1.w);
+    }
+    part[h] = (q[0] + q[1]) + (q[2] + q[3]);
+  }
+  // Position p of a fragment holds sub-block GX_PERM[p] = {0, 2, 1, 3, 4, 6, 5, 7}[p], its own inverse.
+  auto put = [&](int c, int i, int h, float y) {
+    const int p = (c & 4) | ((c & 1) << 1) | ((c >> 1) & 1);
+    *reinterpret_cast<_Float16*>(sums(i, h) + 2 * p) = (_Float16)y;
+  };
+  if constexpr (SUMS == 1) {
+    const float y = (part[0] + part[1]) * XSUM_UNIT, hi = (float)(_Float16)y;
+    put(u, 0, 0, hi);
+    put(u, 0, 1, y - hi);
+  }
+  if constexpr (SUMS == 2)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int c = 2 * u + h;
+      const float y = part[h] * XSUM_UNIT, hi = (float)(_Float16)y;
+      put(c & 7, 0, c >> 3, hi);
+      put(c & 7, 1, c >> 3, y - hi);
+    }
+}
+
 // ---- activations: global -> LDS ---------------------------------------------
 //
-// global_load_lds_dwordx4 moves 16 bytes per lane into LDS (lane l's at M0 +
-// 16 l) without passing through registers.  The loads are counted by hand
-// (the compiler does not see that they write LDS): loads return in order, so a
-// wait for at most n outstanding ones covers every load with n later ones, and
-// a barrier then covers the other waves'.
-__device__ __forceinline__ void gx_dma16(const uint8_t* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+// buffer_load ... lds moves 16 (or 4) bytes per lane into LDS (lane l's at the
+// wave-uniform destination + 16 l) without passing through registers.  Loads
+// return in order, so a wait for at most n outstanding ones covers every load
+// with n later ones, and a barrier then covers the other waves'.  Buffer loads,
+// because the compiler counts those exactly: after a global_load_lds it waits
+// for every outstanding load before it uses any loaded weight.
+typedef __amdgpu_buffer_rsrc_t gx_rsrc;
+__device__ __forceinline__ gx_rsrc gx_buffer(const uint8_t* base, size_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(base), (short)0, (int)(uint32_t)bytes, 0x00020000);
+}
+__device__ __forceinline__ void gx_dma16(gx_rsrc r, uint32_t lane_off, uint32_t off, uint32_t lds) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(uintptr_t)lds, 16, lane_off, off, 0, 0);
+}
+__device__ __forceinline__ void gx_dma4(gx_rsrc r, uint32_t lane_off, uint32_t off, uint32_t lds) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(uintptr_t)lds, 4, lane_off, off, 0, 0);
+}
+// At most N of this wave's global loads outstanding, its LDS accesses done,
+// then the workgroup's barrier.
+template <int N>
+__device__ __forceinline__ void gx_wait_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p;
 }
-template <class T>
-__device__ __forceinline__ const T* uniform_ptr(const T* p) {
-  const uint64_t v = (uint64_t)(uintptr_t)p;
-  return (const T*)(uintptr_t)(((uint64_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
-                               (uint32_t)__builtin_amdgcn_readfirstlane((int)v));
-}
+// Where a workgroup's activations come from: fragment f (0..31) and aux
+// fragment i (0: the 32 vectors' 1 / S, then the sums) of vector block v in
+// column s, moved into LDS at dst.
+//
+// GxDense: images of whole 32-vector blocks.
+template <int NV> struct GxDense {
+  gx_rsrc img[NV];
+  uint32_t lo16;  // 16 * lane
+  __device__ __forceinline__ void frag(int v, int s, int f, uint32_t dst) const {
+    gx_dma16(img[v], lo16, s * GX_COL + f * 1024, dst);
+  }
+  __device__ __forceinline__ void aux(int v, int s, int i, uint32_t dst) const {
+    gx_dma16(img[v], lo16, s * GX_COL + GX_AUX + 1024 * i, dst);
+  }
+};
+
+// GxRows: any 32 rows of an image kept row by row (the MoE experts' jobs):
+// record (row, column) holds the 32 fragments' 2 x 16 bytes of its vector (32 f
+// + 16 h), at GX_RAUX the sums in fragment order and at GX_RINV 1 / S.
+constexpr int GX_RAUX = 1024;
+constexpr int GX_RINV = GX_RAUX + 64;
+constexpr int GX_REC = 1152;
+template <int NV> struct GxRows {
+  gx_rsrc img;
+  uint32_t row[NV];  // byte offset of lane l % 32's row in block v
+  uint32_t h16;      // 16 * (lane / 32)
+  __device__ __forceinline__ void frag(int v, int s, int f, uint32_t dst) const {
+    gx_dma16(img, row[v] + h16, s * GX_REC + f * 32, dst);
+  }
+  __device__ __forceinline__ void aux(int v, int s, int i, uint32_t dst) const {
+    if (i == 0) gx_dma4(img, row[v], s * GX_REC + GX_RINV, dst);
+    else gx_dma16(img, row[v] + h16, s * GX_REC + GX_RAUX + 32 * (i - 1), dst);
+  }
+};
 
 // LDS of a workgroup of NV vector blocks: the ring of stages, then two
 // columns' aux (1 / S and the min-term fragments).
 template <int KIND, int NV> struct GxLds {
   static constexpr int AUXB = (1 + gx_sums(KIND)) * 1024;
-  static constexpr int AUX0 = GX_RING * NV * GX_STAGE, BYTES = AUX0 + 2 * NV * AUXB;
+  static constexpr int AUX0 = gx_ring(NV) * NV * GX_STAGE, BYTES = AUX0 + 2 * NV * AUXB;
 };
 
 // The columns [s0, s1) of 32 rows (rows row0 .. of the 64-row tile whose packed
-// columns start at W) against NV 32-vector blocks with images img[v]: acc[v][i]
-// is the sum for row row0 + l % 32 and vector i % 4 + 8 (i / 4) + 4 (l / 32) of
-// block v.  The four waves of the workgroup share the staged activations: all
-// call this with the same s0 < s1 and img; W, row0 and img are wave-uniform.
+// columns start at W) against NV 32-vector blocks of X: acc[v][i] is the sum for
+// row row0 + l % 32 and vector i % 4 + 8 (i / 4) + 4 (l / 32) of block v.  The
+// four waves of the workgroup share the staged activations: all call this with
+// the same s0 < s1 and X; W, row0 and X's bases are wave-uniform.
 //
 // 32 rows x 64 vectors a wave: a weight fragment is decoded once for four
 // MFMAs (six for Q6_K).  With two waves per SIMD a wave issues a vector
 // instruction every ~8 cycles and an MFMA takes 32, so the vector instructions
 // per MFMA set the time: a loop of MFMAs alone runs at 14.2 ns each, with 6
 // vector instructions each at 17.5, with 10 at 24 ns.
-template <int KIND, int NV>
-__device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, int s1, const uint8_t* const (&img)[NV],
-                                           uint8_t* lds, f16v (&acc)[NV]) {
+template <int KIND, int NV, class SRC>
+__device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, int s1, const SRC& X, uint8_t* lds,
+                                           f16v (&acc)[NV]) {
   using U = GxW<KIND>;
   using L = GxLds<KIND, NV>;
   constexpr int SUMS = gx_sums(KIND), GB = U::GB, AUXN = 1 + SUMS;
   const int lane = threadIdx.x & 63, h = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t ring = __builtin_amdgcn_readfirstlane(lds_offset(lds)), lo16 = 16 * lane;
+  constexpr int R = gx_ring(NV);
+  // Loads a wave issues per R - 2 consecutive stages: the fragments, and the
+  // body loads (one per stage, two for Q8_0, three in every other one for Q6_K,
+  // one in every other one for Q2_K and Q3_K).
+  constexpr int DMA = (R - 2) * 2 * NV;
+  constexpr int BODY = (R - 2) * (KIND == Q8_0 ? 4 : KIND == Q6_K ? 3 : KIND == Q2_K || KIND == Q3_K ? 1 : 2) / 2;
   const int last = 4 * (s1 - s0) - 1;  // stages
   // Stage g's 8 NV fragments, 2 NV per wave (past the end the last stage
   // again, into a slot nobody reads, so that every stage issues as many).
-  auto dma_stage = [&](int g) {
+  auto dma_stage = [&](int g, int slot) {
     const int c = g < last ? g : last;
-    const size_t off = (size_t)(s0 + (c >> 2)) * GX_COL + ((c & 3) * 8 + 2 * w) * 1024;
-    const uint32_t dst = ring + (g % GX_RING) * NV * GX_STAGE + 2 * w * 1024;
+    const int s = s0 + (c >> 2), f = (c & 3) * 8 + 2 * w;
+    const uint32_t dst = ring + slot * NV * GX_STAGE + 2 * w * 1024;
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-      gx_dma16(img[v] + off, lo16, dst + v * GX_STAGE);
-      gx_dma16(img[v] + off + 1024, lo16, dst + v * GX_STAGE + 1024);
+      X.frag(v, s, f, dst + v * GX_STAGE);
+      X.frag(v, s, f + 1, dst + v * GX_STAGE + 1024);
     }
   };
   auto dma_aux = [&](int c) {  // of column s0 + c, one fragment per wave in turn
-    const size_t off = (size_t)min(s0 + c, s1 - 1) * GX_COL + GX_AUX;
+    const int s = min(s0 + c, s1 - 1);
     const uint32_t dst = ring + L::AUX0 + (c & 1) * NV * L::AUXB;
 #pragma unroll
     for (int v = 0; v < NV; ++v)
 #pragma unroll
       for (int i = 0; i < AUXN; ++i)
-        if (((v * AUXN + i) & 3) == w) gx_dma16(img[v] + off + 1024 * i, lo16, dst + v * L::AUXB + 1024 * i);
+        if (((v * AUXN + i) & 3) == w) X.aux(v, s, i, dst + v * L::AUXB + 1024 * i);
   };
   const int row = row0 + (lane & 31), ro = 16 * row;
   U wt;
   const uint8_t* g0 = W + (size_t)s0 * GB;
+  dma_aux(0);
+#pragma unroll
+  for (int g = 0; g < R - 1; ++g) dma_stage(g, g);
   wt.load_head(g0, row, ro, h);
 #pragma unroll
   for (int j = 0; j < 4; ++j) wt.load_body(g0, ro, h, j);
-  dma_aux(0);
-#pragma unroll
-  for (int g = 0; g < GX_RING - 1; ++g) dma_stage(g);
+  // All of them (vmcnt 0): the loop's waits then count from here on both paths
+  // into it, the compiler's for the weights as well as those below.
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  asm volatile("" ::: "memory");
+  int slot = 0, fill = R - 1;  // this stage's slot, the next one to fill
   f16v sum[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) sum[v] = acc[v] = zero16();
@@ -406,11 +527,11 @@ __device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, i
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int g = 4 * c + j;
-      // This wave's loads of stage g are done (stages g + 1 and g + 2 issued
-      // 4 NV later ones) and its reads of stage g - 1; then everyone's.
-      if constexpr (NV == 2) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      const uint8_t* st = lds + (g % GX_RING) * NV * GX_STAGE + lo16;
+      // This wave's loads of stage g are done (the R - 2 stages issued after it
+      // count DMA + BODY later ones) and its reads of stage g - 1; then
+      // everyone's.
+      gx_wait_barrier<DMA + BODY>();
+      const uint8_t* st = lds + slot * NV * GX_STAGE + lo16;
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const int u = 2 * j + t;
@@ -457,7 +578,9 @@ __device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, i
       }
       wt.load_body(g0, ro, h, j);
       if (j == 1) dma_aux(c + 1);
-      dma_stage(g + GX_RING - 1);
+      dma_stage(g + R - 1, fill);
+      slot = slot + 1 == R ? 0 : slot + 1;
+      fill = fill + 1 == R ? 0 : fill + 1;
     }
     // The column's d, mins and 1 / S.
     const uint8_t* ax = lds + L::AUX0 + (c & 1) * NV * L::AUXB;

@@ -9,7 +9,7 @@
 //                 with the columns split, the last workgroup adds the sums
 //
 // Bound by the matrix cores and the vector instructions around them: Q4_K
-// 28672x4096 x 512 takes 268 us, 0.90 PFLOP/s of f16 MFMA (hi and lo; a plain
+// 28672x4096 x 512 takes 251 us, 0.96 PFLOP/s of f16 MFMA (hi and lo; a plain
 // f16 library product of the same MFMA work reaches 1.05), where eight launches
 // of the 64-vector kernel took 546; Q6_K 5001x3584 x 333 51 us (457 on the
 // one-pass kernel, 32 vectors a launch), Q6_K 4096x14336 x 64 40 us (115), Q5_K
@@ -33,62 +33,9 @@ __global__ __launch_bounds__(256) void kq_gx_split(const float* __restrict__ X, 
   const int m = threadIdx.x >> 3, u = threadIdx.x & 7, nsb = in_dim / 256;
   const int s = blockIdx.x, row = blockIdx.y * 32 + m;
   uint8_t* out = img + ((size_t)blockIdx.y * nsb + s) * GX_COL;
-  float4 v[8];
-  const float4* src = reinterpret_cast<const float4*>(X + (size_t)row * in_dim + 256 * s + 32 * u);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = row < B ? src[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-  float a = 0.f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) a = fmaxf(a, fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w))));
-#pragma unroll
-  for (int o = 1; o < 8; o <<= 1) a = fmaxf(a, __shfl_xor(a, o, 64));
-  // S = 2^(14 - e) with a < 2^e, at most 2^116; 1 for zero or non-finite columns.
-  int e = 0;
-  const bool scaled = a > 0.f && __builtin_isfinite(a);
-  if (scaled) (void)frexpf(a, &e);
-  const int ex = scaled ? min(14 - e, 116) : 0;
-  const float S = ldexpf(1.f, ex);
-  if (u == 0) *reinterpret_cast<float*>(out + GX_AUX + 4 * m) = ldexpf(1.f, -ex);
-  float part[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    float q[4];
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      float4 x0 = v[4 * h + 2 * b], x1 = v[4 * h + 2 * b + 1];
-      x0.x *= S; x0.y *= S; x0.z *= S; x0.w *= S;
-      x1.x *= S; x1.y *= S; x1.z *= S; x1.w *= S;
-      const h8 hi = {(_Float16)x0.x, (_Float16)x0.z, (_Float16)x0.y, (_Float16)x0.w,
-                     (_Float16)x1.x, (_Float16)x1.z, (_Float16)x1.y, (_Float16)x1.w};
-      const h8 lo = {(_Float16)(x0.x - (float)hi[0]), (_Float16)(x0.z - (float)hi[1]), (_Float16)(x0.y - (float)hi[2]),
-                     (_Float16)(x0.w - (float)hi[3]), (_Float16)(x1.x - (float)hi[4]), (_Float16)(x1.z - (float)hi[5]),
-                     (_Float16)(x1.y - (float)hi[6]), (_Float16)(x1.w - (float)hi[7])};
-      uint8_t* f = out + (4 * u + 2 * b) * 1024 + (h * 32 + m) * 16;
-      *reinterpret_cast<h8*>(f) = hi;
-      *reinterpret_cast<h8*>(f + 1024) = lo;
-      q[2 * b] = (x0.x + x0.y) + (x0.z + x0.w);
-      q[2 * b + 1] = (x1.x + x1.y) + (x1.z + x1.w);
-    }
-    part[h] = (q[0] + q[1]) + (q[2] + q[3]);
-  }
-  // Position p of a fragment holds sub-block GX_PERM[p] = {0, 2, 1, 3, 4, 6, 5, 7}[p], its own inverse.
-  auto put = [&](int c, int frag, int half, float x) {
-    const int p = (c & 4) | ((c & 1) << 1) | ((c >> 1) & 1);
-    *reinterpret_cast<_Float16*>(out + GX_SUM + frag * 1024 + (half * 32 + m) * 16 + 2 * p) = (_Float16)x;
-  };
-  if constexpr (SUMS == 1) {
-    const float x = (part[0] + part[1]) * XSUM_UNIT, hi = (float)(_Float16)x;
-    put(u, 0, 0, hi);
-    put(u, 0, 1, x - hi);
-  }
-  if constexpr (SUMS == 2)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int c = 2 * u + h;
-      const float x = part[h] * XSUM_UNIT, hi = (float)(_Float16)x;
-      put(c & 7, 0, c >> 3, hi);
-      put(c & 7, 1, c >> 3, x - hi);
-    }
+  gx_split<SUMS>(row < B ? X + (size_t)row * in_dim + 256 * s : nullptr, u,
+                 [&](int f, int h) { return out + f * 1024 + (h * 32 + m) * 16; },
+                 [&](int i, int h) { return out + GX_SUM + i * 1024 + (h * 32 + m) * 16; }, out + GX_AUX + 4 * m);
 }
 
 struct GemmArgs {
@@ -114,11 +61,12 @@ __global__ __launch_bounds__(256, NV == 1 ? 3 : 2) void kq_gemm(GemmArgs a) {
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int want = 2 * group + (w >> 1), tile = min(want, a.tiles - 1), row0 = 32 * (w & 1);
   const size_t vstride = (size_t)a.nsb * GX_COL;
-  const uint8_t* img[NV];
+  GxDense<NV> X;
 #pragma unroll
-  for (int v = 0; v < NV; ++v) img[v] = a.img + min(NV * vg + v, a.vblocks - 1) * vstride;
+  for (int v = 0; v < NV; ++v) X.img[v] = gx_buffer(a.img + min(NV * vg + v, a.vblocks - 1) * vstride, vstride);
+  X.lo16 = 16 * lane;
   f16v acc[NV];
-  gx_columns<KIND, NV>(a.P + (size_t)tile * a.nsb * GxW<KIND>::GB, row0, s0, s1, img, lds, acc);
+  gx_columns<KIND, NV>(a.P + (size_t)tile * a.nsb * GxW<KIND>::GB, row0, s0, s1, X, lds, acc);
   // Columns split over ks workgroups: each stores its sums (a tile's as
   // [v][i / 2][thread] pairs), the last to arrive adds the ks of them in
   // ascending order.  Agent-scope accesses and a counter, no fence, as in
