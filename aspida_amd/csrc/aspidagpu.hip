@@ -1061,10 +1061,9 @@ static int moe_chunk(int T, int top_k) { return std::min(T, kq::MOE_MAX_JOBS / t
 extern "C" long aspida_moe_packed_work_bytes(int T, int dim, int intermed, int top_k) {
   if (T <= 0 || dim <= 0 || intermed <= 0 || top_k <= 0 || top_k > kq::MOE_MAX_TOPK) return -EINVAL;
   size_t n = kq::moe_grouped_work_bytes(moe_chunk(T, top_k), dim, intermed, top_k);
-  // From MOE_PREFILL_MIN_TOKENS tokens the Q4_K / Q6_K experts may take the
-  // prefill products, in launch sequences of up to MOE_PREFILL_MAX_TOKENS.
-  if (T >= kq::MOE_PREFILL_MIN_TOKENS && dim % 256 == 0 && intermed % 256 == 0)
-    n = std::max(n, kq::moe_prefill_work_bytes(std::min(T, kq::MOE_PREFILL_MAX_TOKENS), dim, intermed, top_k));
+  // The experts may take the grouped products, in launch sequences of up to
+  // MOE_PREFILL_MAX_TOKENS.
+  n = std::max(n, kq::moe_prefill_work_bytes(T, dim, intermed, top_k));
   return (long)n;
 }
 
@@ -1119,18 +1118,27 @@ int kq::moe_experts_packed_norm(const float* x, int T, int dim, int top_k, int i
   a.d_stride = kq::packed_bytes(down_kind, intermed, dim);
   a.sgi = shared_gate_inp;
   a.top_k = top_k; a.n_exp = n_exp; a.dim = dim; a.I = intermed;
-  if (kq::moe_prefill_takes(T, gu_kind, down_kind, dim, intermed, top_k, n_exp) && kq::matvec_mfma_takes(gu_kind) &&
-      kq::matvec_mfma_takes(down_kind)) {
-    // Many tokens: the grouped products of kq_moe_prefill.hip, in sequences of
-    // up to MOE_PREFILL_MAX_TOKENS tokens (a last short one included).
+  if (kq::moe_prefill_takes(T, gu_kind, down_kind, dim, intermed, top_k, n_exp) && kq::matvec_engine() == 0) {
+    // The grouped products of kq_moe_prefill.hip, in sequences of up to
+    // MOE_PREFILL_MAX_TOKENS tokens (a last short one included).
     for (int t0 = 0; t0 < T; t0 += kq::MOE_PREFILL_MAX_TOKENS) {
       a.T = std::min(kq::MOE_PREFILL_MAX_TOKENS, T - t0);
       a.x = x + (size_t)t0 * dim;
       a.idx = top_idx + (size_t)t0 * top_k;
       a.top_w = top_w + (size_t)t0 * top_k;
       a.y = y + (size_t)t0 * dim;
-      const int rc = check(kq::launch_moe_prefill(a, work, (hipStream_t)stream), "aspida_moe_experts_packed_dev");
+      // The norm goes into the combine only when one sequence covers the tokens.
+      bool done = false;
+      if (norm_h && norm_w && norm_nx && T <= kq::MOE_PREFILL_MAX_TOKENS) {
+        a.norm_h = norm_h;
+        a.norm_w = norm_w;
+        a.norm_nx = norm_nx;
+        a.norm_done = &done;
+      }
+      const int rc = check(kq::launch_moe_prefill(a, gu_kind, down_kind, work, (hipStream_t)stream),
+                           "aspida_moe_experts_packed_dev");
       if (rc) return rc;
+      if (norm_done) *norm_done = done;
     }
     return 0;
   }

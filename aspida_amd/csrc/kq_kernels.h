@@ -149,6 +149,7 @@ hipError_t launch_pack(int kind, const void* src, int in_dim, int out_dim, void*
 // takes.  set_matvec_engine(1) keeps every kind on the VALU kernel
 // (comparison), 0 restores the default.
 void set_matvec_engine(int engine);
+int matvec_engine();
 bool matvec_mfma_takes(int kind);
 // The 16-row matrix-core matvec with its x formed in the launch: x =
 // RMSNorm(H + r) with weights g (r may be null; H is not written).  Q4_K and

@@ -1,6 +1,5 @@
 // kq_mmq.h -- the matrix-core arithmetic of the small-batch K-quant products
-// (kq_mmq.hip), shared with the grouped MoE prefill products
-// (kq_moe_prefill.hip): the activation split, the activation tiles staged in
+// (kq_mmq.hip): the activation split, the activation tiles staged in
 // LDS, and one super-block column of Q4_K or Q6_K weights multiplied against
 // such a tile.  Numerics and MFMA lane layouts: the notes at the top of
 // kq_mmq.hip.

@@ -114,17 +114,19 @@ hipError_t launch_moe_grouped_mfma(const MoeGroupedArgs& a, int gu_kind, int dow
 
 // ---- prefill: many tokens per launch (kq_moe_prefill.hip) ----
 
-// Tokens from which Q4_K gate/up with Q6_K down run the grouped GEMM of
-// kq_moe_prefill.hip, and the most tokens one of its launch sequences takes.
-constexpr int MOE_PREFILL_MIN_TOKENS = 96;  // measured: 64 tokens 256 us here vs 239 us grouped
+// Where the experts run as the grouped products of kq_moe_prefill.hip, and the
+// most tokens one of its launch sequences takes.
 constexpr int MOE_PREFILL_MAX_TOKENS = 1024;
 bool moe_prefill_takes(int T, int gu_kind, int down_kind, int dim, int I, int top_k, int n_exp);
-// Work bytes of one launch sequence of T <= MOE_PREFILL_MAX_TOKENS tokens
-// (any n_exp up to MOE_MAX_EXP).
+// Work bytes of its launch sequences for T tokens (any n_exp up to
+// MOE_MAX_EXP), 0 where no shape takes it.
 size_t moe_prefill_work_bytes(int T, int dim, int I, int top_k);
-// a: the weights, idx, top_w, x, sgi, y, T, top_k, n_exp, dim, I of
-// MoeGroupedArgs (its work pointers are not used); work 256-byte aligned.
-hipError_t launch_moe_prefill(const MoeGroupedArgs& a, void* work, hipStream_t s);
+// a: the weights, idx, top_w, x, sgi, y, norm pointers, T, top_k, n_exp, dim, I
+// of MoeGroupedArgs (its work pointers are not used); work 256-byte aligned.
+hipError_t launch_moe_prefill(const MoeGroupedArgs& a, int gu_kind, int down_kind, void* work, hipStream_t s);
+// The combine of a's slot outputs yk and gates gsh into y (kq_moe_mfma.hip),
+// with the model chain's next norm where a asks for it.
+hipError_t launch_moe_combine(const MoeGroupedArgs& a, hipStream_t s);
 
 // Router: logits[t] = router_w[n_exp][dim] . x[t] (f32), stable softmax,
 // greedy top-k (strict >, lowest index wins ties), renormalised weights

@@ -682,10 +682,7 @@ static void launch_down_mf(const MoeGroupedArgs& a, hipStream_t s) {
 
 bool moe_mfma_kind(int kind) { return kind == Q4_K || kind == Q6_K; }
 
-template <int GK, int DK>
-static hipError_t launch_mr(const MoeGroupedArgs& a, hipStream_t s) {
-  launch_gate_up_mf<GK>(a, s);
-  launch_down_mf<DK>(a, s);
+hipError_t launch_moe_combine(const MoeGroupedArgs& a, hipStream_t s) {
   if (a.norm_h && a.norm_w && a.norm_nx && a.dim % 4 == 0) {
     hipLaunchKernelGGL(moe_combine_norm_mf, dim3(a.T), dim3(MR_NORM_THREADS), 0, s, a);
     if (a.norm_done) *a.norm_done = true;
@@ -693,6 +690,13 @@ static hipError_t launch_mr(const MoeGroupedArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(moe_combine_mf, dim3((a.dim + 255) / 256, a.T), dim3(256), 0, s, a);
   }
   return hipGetLastError();
+}
+
+template <int GK, int DK>
+static hipError_t launch_mr(const MoeGroupedArgs& a, hipStream_t s) {
+  launch_gate_up_mf<GK>(a, s);
+  launch_down_mf<DK>(a, s);
+  return launch_moe_combine(a, s);
 }
 
 hipError_t launch_moe_grouped_mfma(const MoeGroupedArgs& a, int gu_kind, int down_kind, hipStream_t s) {

@@ -1,74 +1,65 @@
-// kq_moe_prefill.hip -- the grouped MoE experts for many tokens at once
-// (prefill chunks) on the matrix cores: a grouped GEMM over the experts'
-// packed Q4_K gate / up and Q6_K down matrices, for Q4_K_M-style layers.
+// kq_moe_prefill.hip -- the grouped MoE experts for several tokens at once as a
+// grouped product over the experts' packed matrices, for every kind, on the
+// arithmetic of kq_gemm.h.
 //
-// Per launch sequence of up to PF_MAX_TOKENS tokens (LLM_MoE.Forward steps 4-5,
-// src/llm/llm_moe.adb:249-299, for every token; the reference's prefill runs
-// K-quant experts per token, gpu/gpu_matvec.cu:4237-4239):
+// Per launch sequence of up to MOE_PREFILL_MAX_TOKENS tokens (LLM_MoE.Forward
+// steps 4-5, src/llm/llm_moe.adb:249-299, for every token; the reference's
+// prefill runs K-quant experts per token, gpu/gpu_matvec.cu:4237-4239):
 //
-//   kq_xsplit<32>   the tokens' activations as f16 hi / lo images (kq_mmq.h)
-//   moe_pf_plan     one workgroup: every (token, slot) job bucketed by expert
-//                   (shared expert first), cut into groups of up to BP jobs
-//   moe_pf_gate_up  per (group, 64-row tile): gate and up rows of the group's
-//                   expert against the group's activation rows, gathered by
-//                   token; h[job][row] = silu(gate) * up
-//   moe_pf_gates    the tokens' shared-expert gates g_t, one wave per token
-//   kq_xsplit<16>   h as f16 hi / lo images, one row per job
-//   moe_pf_down     per (group, 64-row tile of dim): yk[job][row] = down . h[job]
-//   moe_pf_combine  y[t] = sum_k top_w[t][k] yk[t, k] (ascending k) +
-//                   g_t yk[t, shared], g_t = sigmoid(shared_gate_inp . x_t)
-//                   (1 without shared_gate_inp)
+//   moe_gx_prep     block 0: every (token, slot) job bucketed by expert (shared
+//                   expert first), cut into groups of up to BP jobs; the other
+//                   blocks: the tokens' activations as f16 hi / lo records, and
+//                   the shared-expert gates
+//   moe_gx_gate_up  per (group, 64 rows): gate and up rows of the group's expert
+//                   against its jobs' tokens; h[job][row] = silu(gate) * up
+//   moe_gx_hsplit   h as f16 hi / lo records, one row per job
+//   moe_gx_down     per (group, 128 rows of dim): yk[job][row] = down . h[job]
+//   moe_combine_mf  y[t] = sum_k top_w[t][k] yk[t, k] (ascending k) + g_t
+//                   yk[t, shared] (kq_moe_mfma.hip)
 //
-// Each product tile reads its 64 weight rows once for up to BP = 64 jobs, so
-// the weights of an expert are read once per BP of its jobs rather than once
-// per job, and the matrix cores do the f16 products with the small-batch
-// arithmetic (exact integer codes, activations split into hi + lo; kq_mmq.h).
-// Within an expert's bucket the jobs' order is not fixed (atomic placement),
-// but every output element is one job's own dot product over all columns in
-// a fixed order, and the combine sums in ascending k: the results are
-// deterministic.
+// A group's weights are decoded once for all its jobs; a group of up to 32 jobs
+// takes the one-block form of gx_columns, so a short group costs half a full
+// one.  Within an expert's bucket the jobs' order is not fixed (atomic
+// placement), but every output element is one job's own dot product over all
+// columns in a fixed order, and the combine sums in ascending k: the results
+// are deterministic.
+//
+// Bound by the matrix cores and the vector instructions around them (kq_gemm.h)
+// from about 100 tokens, by the weights' latency below.  The Qwen3-MoE layer
+// (2048x768, 128 experts and a shared one, top 8, Q4_K / Q6_K, router included):
+// 1024 tokens 436 us (889 on 16x16x16 products of 64-job tiles), 512 283 (474),
+// 256 200 (352), 128 184 (265), 64 166 (216); Q5_K / Q6_K 256 tokens 205 (1468
+// on the vector ALUs).  At 1024: prep 14, gate/up 234, h split 20, down 156,
+// combine 22.
 #include <math.h>
 
 #include <algorithm>
 
+#include "kq_gemm.h"
 #include "kq_kernels.h"
-#include "kq_mmq.h"
 #include "kq_moe.h"
 
 namespace kq {
 
-struct PfArgs {
-  const uint8_t *gate, *up, *down, *sh_gate, *sh_up, *sh_down;
-  size_t gu_stride, d_stride;
-  const int* idx;
-  const float *top_w, *x, *sgi;
-  float* y;
-  int T, top_k, n_exp, dim, I;
-  // work
-  _Float16 *xh, *xl, *xsh, *xsl;
-  float* xinv;
-  float* gsh;   // [T] shared-expert gates
-  float* h;
-  _Float16 *hh, *hl, *hsh, *hsl;
-  float* hinv;
-  float* yk;
-  int* jobs;    // [T slots]: job = t slots + k, bucketed by expert position
-  int4* units;  // [0].x = group count; [1 + c] = group c: {expert, first job (into jobs), job count, 0}
+struct GxMoe {
+  MoeGroupedArgs g;     // weights, idx, top_w, x, sgi, y, h, yk, gsh
+  uint8_t *ximg, *himg;  // records: [T][dim / 256], [T slots][I / 256]
+  int* jobs;             // [T slots]: job = t slots + k, bucketed by expert position
+  int4* units;           // [0].x = group count; [1 + c] = group c: {expert, first job (into jobs), job count, 0}
 };
 
-__device__ __forceinline__ int pf_expert_at(int p, int n_exp) { return p == 0 ? n_exp : p - 1; }
+__device__ __forceinline__ int gx_expert_at(int p, int n_exp) { return p == 0 ? n_exp : p - 1; }
 
-// ---- plan -------------------------------------------------------------------------
+constexpr int PREP_THREADS = 1024;
 
-template <int BP>
-__global__ __launch_bounds__(1024) void moe_pf_plan(PfArgs a) {
+__device__ __forceinline__ void gx_plan(const GxMoe& a, int BP) {
   __shared__ int cnt[MOE_MAX_EXP + 1], off[MOE_MAX_EXP + 2], coff[MOE_MAX_EXP + 2], cur[MOE_MAX_EXP + 1];
-  const int ne = a.n_exp + 1, n = a.T * a.top_k, slots = a.top_k + 1, tid = threadIdx.x;
-  for (int p = tid; p < ne; p += 1024) cnt[p] = p == 0 ? a.T : 0;
+  const int T = a.g.T, top_k = a.g.top_k, ne = a.g.n_exp + 1, n = T * top_k, slots = top_k + 1, tid = threadIdx.x;
+  for (int p = tid; p < ne; p += PREP_THREADS) cnt[p] = p == 0 ? T : 0;
   __syncthreads();
-  for (int i = tid; i < n; i += 1024) {
-    const int e = a.idx[i];
-    if (e >= 0 && e < a.n_exp) atomicAdd(&cnt[e + 1], 1);
+  for (int i = tid; i < n; i += PREP_THREADS) {
+    const int e = a.g.idx[i];
+    if (e >= 0 && e < a.g.n_exp) atomicAdd(&cnt[e + 1], 1);
   }
   __syncthreads();
   // Exclusive sums of the jobs and of the groups per position (one wave).
@@ -91,15 +82,15 @@ __global__ __launch_bounds__(1024) void moe_pf_plan(PfArgs a) {
     }
   }
   __syncthreads();
-  for (int p = tid; p < ne; p += 1024) cur[p] = off[p] + (p == 0 ? a.T : 0);
+  for (int p = tid; p < ne; p += PREP_THREADS) cur[p] = off[p];
   __syncthreads();
-  for (int t = tid; t < a.T; t += 1024) a.jobs[t] = t * slots + a.top_k;  // position 0: the shared expert
-  for (int i = tid; i < n; i += 1024) {
-    const int e = a.idx[i];
-    if (e >= 0 && e < a.n_exp) a.jobs[atomicAdd(&cur[e + 1], 1)] = (i / a.top_k) * slots + i % a.top_k;
+  for (int t = tid; t < T; t += PREP_THREADS) a.jobs[t] = t * slots + top_k;  // position 0: the shared expert
+  for (int i = tid; i < n; i += PREP_THREADS) {
+    const int e = a.g.idx[i];
+    if (e >= 0 && e < a.g.n_exp) a.jobs[atomicAdd(&cur[e + 1], 1)] = (i / top_k) * slots + i % top_k;
   }
   const int groups = coff[ne];
-  for (int c = tid; c < groups; c += 1024) {
+  for (int c = tid; c < groups; c += PREP_THREADS) {
     int lo = 0, hi = ne - 1;  // the position p with coff[p] <= c < coff[p + 1]
     while (lo < hi) {
       const int mid = (lo + hi + 1) >> 1;
@@ -107,391 +98,278 @@ __global__ __launch_bounds__(1024) void moe_pf_plan(PfArgs a) {
       else hi = mid - 1;
     }
     const int k = c - coff[lo];
-    a.units[1 + c] = make_int4(pf_expert_at(lo, a.n_exp), off[lo] + k * BP, std::min(BP, cnt[lo] - k * BP), 0);
+    a.units[1 + c] = make_int4(gx_expert_at(lo, a.g.n_exp), off[lo] + k * BP, min(BP, cnt[lo] - k * BP), 0);
   }
   if (tid == 0) a.units[0] = make_int4(groups, 0, 0, 0);
 }
 
-// ---- products ---------------------------------------------------------------------
-
-// Thread t's share of column s's activation tile, its rows gathered: tile
-// row b is row rows[b] of the split images (kq_mmq.h, XTile).
-template <int MB>
-__device__ __forceinline__ void pf_xload(const _Float16* xh, const _Float16* xl, const _Float16* sh, const _Float16* sl,
-                                         int nsb, const int* rows, int s, xu4 (&v)[XTile<MB>::NX], xu4& sv) {
-  const int t = threadIdx.x, in_dim = nsb * 256;
-#pragma unroll
-  for (int u = 0; u < XTile<MB>::NX; ++u) {
-    const int i = t + 256 * u, b = i >> 6, part = i & 63;
-    const _Float16* src = (part < 32 ? xh : xl) + (size_t)rows[b] * in_dim + (size_t)s * 256 + 8 * (part & 31);
-    v[u] = *reinterpret_cast<const xu4*>(src);
-  }
-  const int b = (t >> 2) & (XTile<MB>::BP - 1), part = t & 3;
-  const _Float16* src = (part < 2 ? sh : sl) + ((size_t)rows[b] * nsb + s) * 16 + 8 * (part & 1);
-  sv = *reinterpret_cast<const xu4*>(src);
+// Thread u of row `row`, column s of a record image.
+template <int SUMS>
+__device__ __forceinline__ void gx_record(const float* x, uint8_t* rec, int u) {
+  gx_split<SUMS>(x, u, [&](int f, int h) { return rec + f * 32 + h * 16; },
+                 [&](int i, int h) { return rec + GX_RAUX + i * 32 + h * 16; }, rec + GX_RINV);
 }
 
-// The group of unit u (tiles per group): false when u lies past the plan's
-// groups.  Fills jb (the group's jobs, -1 past its count) and rows (the
-// activation row of each tile row: the job's token for gate / up, the job
-// for down; row 0 past the count).
-template <int BP>
-__device__ __forceinline__ bool pf_group(const PfArgs& a, int c, bool by_token, int* jb, int* rows, int4& G) {
-  if (c >= a.units[0].x) return false;
-  G = a.units[1 + c];
-  const int t = threadIdx.x;
-  if (t < BP) {
-    const int j = t < G.z ? a.jobs[G.y + t] : -1;
-    jb[t] = j;
-    rows[t] = j < 0 ? 0 : by_token ? j / (a.top_k + 1) : j;
+// The plan, the token records and the shared-expert gates g_t = sigmoid(sgi .
+// x_t), or 1 without sgi (llm_moe.adb:285-293), are independent: one launch.
+template <int SUMS>
+__global__ __launch_bounds__(PREP_THREADS) void moe_gx_prep(GxMoe a, int BP, int split_blocks) {
+  if (blockIdx.x == 0) {
+    gx_plan(a, BP);
+    return;
   }
+  const int T = a.g.T, nd = a.g.dim / 256, b = blockIdx.x - 1;
+  if (b < split_blocks) {
+    const int q = b * (PREP_THREADS / 8) + (threadIdx.x >> 3), row = q / nd, s = q % nd;
+    if (row < T)
+      gx_record<SUMS>(a.g.x + (size_t)row * a.g.dim + 256 * s, a.ximg + (size_t)q * GX_REC, threadIdx.x & 7);
+    return;
+  }
+  const int t = (b - split_blocks) * (PREP_THREADS / 64) + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (t >= T) return;
+  float s = 0.f;
+  if (a.g.sgi) {
+    const float4* g4 = reinterpret_cast<const float4*>(a.g.sgi);
+    const float4* x4 = reinterpret_cast<const float4*>(a.g.x + (size_t)t * a.g.dim);
+    for (int i = lane; i < a.g.dim / 4; i += 64) {
+      const float4 gv = g4[i], xv = x4[i];
+      s = __builtin_fmaf(gv.x, xv.x, s);
+      s = __builtin_fmaf(gv.y, xv.y, s);
+      s = __builtin_fmaf(gv.z, xv.z, s);
+      s = __builtin_fmaf(gv.w, xv.w, s);
+    }
+    s = wave_total(s);
+  }
+  if (lane == 0) a.g.gsh[t] = a.g.sgi ? 1.0f / (1.0f + expf(-s)) : 1.0f;
+}
+
+template <int SUMS>
+__global__ __launch_bounds__(256) void moe_gx_hsplit(GxMoe a, int rows) {
+  const int ni = a.g.I / 256, q = blockIdx.x * 32 + (threadIdx.x >> 3), row = q / ni, s = q % ni;
+  if (row < rows) gx_record<SUMS>(a.g.h + (size_t)row * a.g.I + 256 * s, a.himg + (size_t)q * GX_REC, threadIdx.x & 7);
+}
+
+// The unit of workgroup b among N (groups times tiles): the shared expert's S
+// first, dealt over the XCDs (workgroup b runs on XCD b % 8), then each XCD a
+// run of consecutive units, so that the groups of one expert, which read the
+// same weights, share an L2.  -1: none.
+__device__ __forceinline__ int gx_unit(int b, int N, int S) {
+  const int S8 = (S + 7) & ~7;
+  if (b < S8) return b < S ? b : -1;
+  const int per = (N - S + 7) >> 3, x = (b - S8) & 7, l = (b - S8) >> 3, u = S + x * per + l;
+  return l < per && u < N ? u : -1;
+}
+
+template <int NV>
+__device__ __forceinline__ GxRows<NV> gx_rows(const uint8_t* img, int rows, const int* list, const int4& G, int div,
+                                              uint32_t stride, int lane) {
+  GxRows<NV> X;
+  X.img = gx_buffer(img, (size_t)rows * stride);
+  X.h16 = 16 * (lane >> 5);
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {  // past the group: its first job again
+    const int k = 32 * v + (lane & 31);
+    X.row[v] = (uint32_t)(list[G.y + (k < G.z ? k : 0)] / div) * stride;
+  }
+  return X;
+}
+
+// Waves 0 and 2 take the gate's, 1 and 3 the up projection's rows 0..31 and
+// 32..63 of a tile; the up sums meet the gate's in LDS.
+template <int KIND, int NV>
+__device__ __forceinline__ void gx_gate_up(const GxMoe& a, const int4& G, int tile, uint8_t* lds, const int* jb) {
+  const int nsb = a.g.dim / 256, slots = a.g.top_k + 1;
+  const int lane = threadIdx.x & 63, n = lane & 31, h = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), up = w & 1, rb = w >> 1;
+  const int e = __builtin_amdgcn_readfirstlane(G.x);
+  const uint8_t* W = e == a.g.n_exp ? (up ? a.g.sh_up : a.g.sh_gate)
+                                    : (up ? a.g.up : a.g.gate) + (size_t)e * a.g.gu_stride;
+  const GxRows<NV> X = gx_rows<NV>(a.ximg, a.g.T, a.jobs, G, slots, (uint32_t)nsb * GX_REC, lane);
+  f16v acc[NV];
+  gx_columns<KIND, NV>(W + (size_t)tile * nsb * GxW<KIND>::GB, 32 * rb, 0, nsb, X, lds, acc);
   __syncthreads();
-  return true;
-}
-
-// The shared-expert gates g_t = sigmoid(sgi . x_t), or 1 without sgi
-// (llm_moe.adb:285-293), one wave per token.  A launch of its own: inside the
-// gate/up kernel its registers cost the 32-job variant its second wave per
-// SIMD (T = 512: 470 -> 541 us per layer).
-__global__ __launch_bounds__(256) void moe_pf_gates(PfArgs a) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  for (int t = blockIdx.x * 4 + w; t < a.T; t += gridDim.x * 4) {
-    float s = 0.f;
-    if (a.sgi) {
-      const float4* g4 = reinterpret_cast<const float4*>(a.sgi);
-      const float4* x4 = reinterpret_cast<const float4*>(a.x + (size_t)t * a.dim);
-      for (int i = lane; i < a.dim / 4; i += 64) {
-        const float4 gv = g4[i], xv = x4[i];
-        s = __builtin_fmaf(gv.x, xv.x, s);
-        s = __builtin_fmaf(gv.y, xv.y, s);
-        s = __builtin_fmaf(gv.z, xv.z, s);
-        s = __builtin_fmaf(gv.w, xv.w, s);
-      }
-      s = wave_total(s);
-    }
-    if (lane == 0) a.gsh[t] = a.sgi ? 1.0f / (1.0f + expf(-s)) : 1.0f;
-  }
-}
-
-// Gate and up of one (group, 64-row tile): wave w takes rows 16 w .. 16 w + 15
-// of both matrices (acc[0] gate, acc[1] up) over every column.
-template <int MB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void moe_pf_gate_up(PfArgs a) {
-  constexpr int GB = 64 * 144, BP = 16 * MB;
-  __shared__ __attribute__((aligned(16))) _Float16 xb[2][BP * XROW];
-  __shared__ __attribute__((aligned(16))) _Float16 sb[2][BP * SROW];
-  __shared__ int jb[BP], rows[BP];
-  const int tiles = a.I / 64, nsb = a.dim / 256;
-  const int c = blockIdx.x / tiles, tile = blockIdx.x % tiles;
-  int4 G;
-  if (!pf_group<BP>(a, c, true, jb, rows, G)) return;
-  const int lane = threadIdx.x & 63, j = lane & 15, q = lane >> 4;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int e = G.x, row = 16 * w + j;
-  const uint8_t* Wg = (e == a.n_exp ? a.sh_gate : a.gate + (size_t)e * a.gu_stride) + (size_t)tile * nsb * GB;
-  const uint8_t* Wu = (e == a.n_exp ? a.sh_up : a.up + (size_t)e * a.gu_stride) + (size_t)tile * nsb * GB;
-  auto load_w = [&](int s, Q4Regs (&r)[2]) {
-    q4k_load(Wg + (size_t)s * GB, row, q, false, r[0]);
-    q4k_load(Wu + (size_t)s * GB, row, q, false, r[1]);
-  };
-  f4 acc[2][MB];
+  float* xch = reinterpret_cast<float*>(lds) + rb * NV * 16 * 64 + lane;
+  if (up)
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
+    for (int v = 0; v < NV; ++v)
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) acc[rb][mb] = f4{0.f, 0.f, 0.f, 0.f};
-  Q4Regs cur[2], nxt[2];
-  xu4 xv[XTile<MB>::NX], xsv;
-  load_w(0, cur);
-  pf_xload<MB>(a.xh, a.xl, a.xsh, a.xsl, nsb, rows, 0, xv, xsv);
-  xtile_store<MB>(xb[0], sb[0], xv, xsv);
+      for (int i = 0; i < 16; ++i) xch[(v * 16 + i) * 64] = acc[v][i];
   __syncthreads();
-  for (int s = 0; s < nsb; ++s) {
-    const int buf = s & 1;
-    const bool more = s + 1 < nsb;
-    if (more) {
-      load_w(s + 1, nxt);
-      pf_xload<MB>(a.xh, a.xl, a.xsh, a.xsl, nsb, rows, s + 1, xv, xsv);
-    }
-    q4k_column<MB, 2>(cur, xb[buf], sb[buf], j, q, acc);
-    if (more) {
-      xtile_store<MB>(xb[buf ^ 1], sb[buf ^ 1], xv, xsv);
-      cur[0] = nxt[0];
-      cur[1] = nxt[1];
-    }
-    __syncthreads();
-  }
-  // acc[.][mb][r]: activation row b = 16 mb + 4 q + r, weight row `row`.
-  const int orow = 64 * tile + row;
+  if (up) return;
+  float* out = a.g.h + 64 * tile + 32 * rb + n;
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
+  for (int v = 0; v < NV; ++v)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int b = 16 * mb + 4 * q + r, job = jb[b];
-      if (job >= 0) {
-        const float sx = a.xinv[rows[b]];
-        const float g = acc[0][mb][r] * sx, v = acc[1][mb][r] * sx;
-        a.h[(size_t)job * a.I + orow] = (g / (1.0f + expf(-g))) * v;
-      }
+    for (int i = 0; i < 16; ++i) {
+      const int job = jb[32 * v + (i & 3) + 8 * (i >> 2) + 4 * h];
+      const float x = acc[v][i], y = (x / (1.0f + expf(-x))) * xch[(v * 16 + i) * 64];
+      if (job >= 0) out[(size_t)job * a.g.I] = y;
     }
 }
 
-// Down of one (group, 64-row tile of dim): yk[job][row], for groups of up to
-// BPG jobs in passes of 16 MB (the Q6_K column arithmetic at 64 rows would
-// spill registers; the second pass reads the tile's weights from cache).
-template <int MB, int BPG>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void moe_pf_down(PfArgs a) {
-  constexpr int GB = 64 * 210, BP = 16 * MB;
-  __shared__ __attribute__((aligned(16))) _Float16 xb[2][BP * XROW];
-  __shared__ __attribute__((aligned(16))) _Float16 sb[2][BP * SROW];
-  __shared__ int jb[BPG], rows[BPG];
-  const int tiles = a.dim / 64, nsb = a.I / 256;
-  const int c = blockIdx.x / tiles, tile = blockIdx.x % tiles;
-  int4 G;
-  if (!pf_group<BPG>(a, c, false, jb, rows, G)) return;
-  const int lane = threadIdx.x & 63, j = lane & 15, q = lane >> 4;
+template <int KIND, int NV>
+__device__ __forceinline__ void gx_down(const GxMoe& a, const int4& G, int blk, uint8_t* lds, const int* jb) {
+  const int nsb = a.g.I / 256;
+  const int lane = threadIdx.x & 63, n = lane & 31, h = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int e = G.x, row = 16 * w + j;
-  const uint8_t* Wd = (e == a.n_exp ? a.sh_down : a.down + (size_t)e * a.d_stride) + (size_t)tile * nsb * GB;
-  const int orow = 64 * tile + row;
-  for (int base = 0; base < G.z; base += BP) {
-    const int* prow = rows + base;
-    f4 acc[MB];
+  const int e = __builtin_amdgcn_readfirstlane(G.x), tile = 2 * blk + (w >> 1), row0 = 32 * (w & 1);
+  const uint8_t* W = e == a.g.n_exp ? a.g.sh_down : a.g.down + (size_t)e * a.g.d_stride;
+  const GxRows<NV> X = gx_rows<NV>(a.himg, a.g.T * (a.g.top_k + 1), a.jobs, G, 1, (uint32_t)nsb * GX_REC, lane);
+  f16v acc[NV];
+  gx_columns<KIND, NV>(W + (size_t)tile * nsb * GxW<KIND>::GB, row0, 0, nsb, X, lds, acc);
+  float* out = a.g.yk + 64 * tile + row0 + n;
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) acc[mb] = f4{0.f, 0.f, 0.f, 0.f};
-    Q6Regs cur, nxt;
-    xu4 xv[XTile<MB>::NX], xsv;
-    q6k_load(Wd, row, q, cur);
-    pf_xload<MB>(a.hh, a.hl, a.hsh, a.hsl, nsb, prow, 0, xv, xsv);
-    xtile_store<MB>(xb[0], sb[0], xv, xsv);
-    __syncthreads();
-    for (int s = 0; s < nsb; ++s) {
-      const int buf = s & 1;
-      const bool more = s + 1 < nsb;
-      if (more) {
-        q6k_load(Wd + (size_t)(s + 1) * GB, row, q, nxt);
-        pf_xload<MB>(a.hh, a.hl, a.hsh, a.hsl, nsb, prow, s + 1, xv, xsv);
-      }
-      q6k_column<MB>(cur, xb[buf], sb[buf], j, q, acc);
-      if (more) {
-        xtile_store<MB>(xb[buf ^ 1], sb[buf ^ 1], xv, xsv);
-        cur = nxt;
-      }
-      __syncthreads();
+  for (int v = 0; v < NV; ++v)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int job = jb[32 * v + (i & 3) + 8 * (i >> 2) + 4 * h];
+      if (job >= 0) out[(size_t)job * a.g.dim] = acc[v][i];
     }
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int b = base + 16 * mb + 4 * q + r, job = b < BPG ? jb[b] : -1;
-        if (job >= 0) a.yk[(size_t)job * a.dim + orow] = acc[mb][r] * a.hinv[job];
-      }
-  }
 }
 
-// Down for intermediate sizes of at most PF_DN_COLS super-block columns: the
-// group's activations for every column are staged in LDS once per pass of
-// 16 MB jobs, then the workgroup walks PF_DN_TILES 64-row tiles of dim
-// against them -- the next tile's weights in flight while the current one is
-// multiplied, and no barrier between tiles.
-constexpr int PF_DN_COLS = 3;
-constexpr int PF_DN_TILES = 8;
-
-template <int MB, int BPG>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void moe_pf_down_wide(PfArgs a) {
-  constexpr int GB = 64 * 210, BP = 16 * MB, NC = PF_DN_COLS;
-  __shared__ __attribute__((aligned(16))) _Float16 xb[NC][BP * XROW];
-  __shared__ __attribute__((aligned(16))) _Float16 sb[NC][BP * SROW];
-  __shared__ int jb[BPG], rows[BPG];
-  const int tiles = a.dim / 64, blocks = (tiles + PF_DN_TILES - 1) / PF_DN_TILES, nsb = a.I / 256;
-  const int c = blockIdx.x / blocks, tb = blockIdx.x % blocks;
-  int4 G;
-  if (!pf_group<BPG>(a, c, false, jb, rows, G)) return;
-  const int lane = threadIdx.x & 63, j = lane & 15, q = lane >> 4;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int e = G.x, row = 16 * w + j;
-  const uint8_t* Wd = e == a.n_exp ? a.sh_down : a.down + (size_t)e * a.d_stride;
-  const int t0 = tb * PF_DN_TILES, t1 = std::min(tiles, t0 + PF_DN_TILES);
-  auto load_tile = [&](int tile, Q6Regs (&r)[NC]) {
-#pragma unroll
-    for (int s = 0; s < NC; ++s)
-      if (s < nsb) q6k_load(Wd + ((size_t)tile * nsb + s) * GB, row, q, r[s]);
-  };
-  for (int base = 0; base < G.z; base += BP) {
-    Q6Regs cur[NC], nxt[NC];
-    load_tile(t0, cur);
-    {
-      xu4 xv[XTile<MB>::NX], xsv;
-#pragma unroll
-      for (int s = 0; s < NC; ++s)
-        if (s < nsb) {
-          pf_xload<MB>(a.hh, a.hl, a.hsh, a.hsl, nsb, rows + base, s, xv, xsv);
-          xtile_store<MB>(xb[s], sb[s], xv, xsv);
-        }
-    }
-    __syncthreads();
-    for (int tile = t0; tile < t1; ++tile) {
-      if (tile + 1 < t1) load_tile(tile + 1, nxt);
-      f4 acc[MB];
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) acc[mb] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < NC; ++s)
-        if (s < nsb) q6k_column<MB>(cur[s], xb[s], sb[s], j, q, acc);
-      const int orow = 64 * tile + row;
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int b = base + 16 * mb + 4 * q + r, job = b < BPG ? jb[b] : -1;
-          if (job >= 0) a.yk[(size_t)job * a.dim + orow] = acc[mb][r] * a.hinv[job];
-        }
-      if (tile + 1 < t1)
-#pragma unroll
-        for (int s = 0; s < NC; ++s) cur[s] = nxt[s];
-    }
-    __syncthreads();  // the next pass overwrites the staged activations
+// NVM = 2: groups of up to 64 jobs; 1: up to 32, at a higher occupancy.
+template <int KIND, int NVM, bool DOWN>
+__global__ __launch_bounds__(256, NVM == 1 && KIND != Q8_0 ? 3 : 2) void moe_gx_expert(GxMoe a, int tiles, int shared_units) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+  __shared__ int jb[32 * NVM];
+  const int u = gx_unit(blockIdx.x, a.units[0].x * tiles, shared_units);
+  if (u < 0) return;
+  const int4 G = a.units[1 + u / tiles];
+  const int tile = u % tiles;
+  if (threadIdx.x < 32 * NVM) jb[threadIdx.x] = (int)threadIdx.x < G.z ? a.jobs[G.y + threadIdx.x] : -1;
+  __syncthreads();
+  if (NVM == 2 && G.z > 32) {
+    if constexpr (DOWN) gx_down<KIND, NVM>(a, G, tile, lds, jb);
+    else gx_gate_up<KIND, NVM>(a, G, tile, lds, jb);
+  } else {
+    if constexpr (DOWN) gx_down<KIND, 1>(a, G, tile, lds, jb);
+    else gx_gate_up<KIND, 1>(a, G, tile, lds, jb);
   }
-}
-
-// y[t][row] = sum_k top_w[t][k] yk[t slots + k][row] (ascending k) +
-// g_t yk[t slots + top_k][row] (llm_moe.adb:270-299), g_t from
-// moe_pf_gates.  Workgroup (i, t): rows 256 i .. 256 i + 255 of token t.  A token
-// with a routed expert outside [0, n_exp) keeps its y unwritten.
-__global__ __launch_bounds__(256) void moe_pf_combine(PfArgs a) {
-  const int t = blockIdx.y, row = blockIdx.x * 256 + threadIdx.x, slots = a.top_k + 1;
-  bool ok = true;
-  for (int k = 0; k < a.top_k; ++k) {
-    const int e = a.idx[(size_t)t * a.top_k + k];
-    ok = ok && e >= 0 && e < a.n_exp;
-  }
-  if (!ok || row >= a.dim) return;
-  const float gs = a.gsh[t];
-  const float* yt = a.yk + (size_t)t * slots * a.dim + row;
-  float acc = 0.f;
-  for (int k0 = 0; k0 < a.top_k; k0 += 8) {
-    float v[8], wk[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int k = k0 + i < a.top_k ? k0 + i : k0;
-      v[i] = yt[(size_t)k * a.dim];
-      wk[i] = a.top_w[(size_t)t * a.top_k + k];
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (k0 + i < a.top_k) acc = acc + wk[i] * v[i];
-  }
-  a.y[(size_t)t * a.dim + row] = acc + gs * yt[(size_t)a.top_k * a.dim];
 }
 
 // ---- host side --------------------------------------------------------------
 
-static size_t pf_round(size_t n) { return (n + 255) / 256 * 256; }
+// Whether T tokens may take this path at all (moe_prefill_takes decides by the
+// kinds and the experts).  Small experts are bound by launches, of which this
+// path has two more: 1024x256, 16 experts, top 2 45 us against 35 at 48 tokens.
+static bool gx_may_take(int T, int dim, int I) {
+  return dim % 256 == 0 && I % 256 == 0 && (T >= 96 || (T >= 4 && (size_t)dim * I >= (size_t)1 << 19));
+}
+
+static size_t gx_round(size_t n) { return (n + 255) / 256 * 256; }
 
 // Groups a plan can produce: ceil(jobs / BP) plus one partial group per
 // non-empty position.
-static size_t pf_max_groups(int T, int top_k, int n_exp, int bp) {
+static size_t gx_max_groups(int T, int top_k, int n_exp, int bp) {
   const size_t jobs = (size_t)T * (top_k + 1);
   return (jobs + bp - 1) / bp + std::min<size_t>((size_t)n_exp, (size_t)T * top_k) + 1;
 }
 
-size_t moe_prefill_work_bytes(int T, int dim, int I, int top_k) {
-  const size_t J = (size_t)T * (top_k + 1), nd = dim / 256, ni = I / 256;
-  size_t n = 0;
-  n += 2 * pf_round((size_t)T * dim * 2);       // xh, xl
-  n += 2 * pf_round((size_t)T * nd * 16 * 2);   // xsh, xsl
-  n += pf_round((size_t)T * 4);                 // xinv
-  n += pf_round((size_t)T * 4);                 // gsh
-  n += pf_round(J * I * 4);                     // h
-  n += 2 * pf_round(J * I * 2);                 // hh, hl
-  n += 2 * pf_round(J * ni * 16 * 2);           // hsh, hsl
-  n += pf_round(J * 4);                         // hinv
-  n += pf_round(J * dim * 4);                   // yk
-  n += pf_round(J * 4);                         // jobs
-  n += pf_round((1 + pf_max_groups(T, top_k, MOE_MAX_EXP, 16)) * 16);  // units (for the smallest groups)
-  return n;
-}
-
-static void pf_bind(PfArgs& a, void* work) {
-  const size_t J = (size_t)a.T * (a.top_k + 1), nd = a.dim / 256, ni = a.I / 256;
-  uint8_t* p = (uint8_t*)work;
+static uint8_t* gx_layout(GxMoe& a, uint8_t* p) {
+  const size_t T = a.g.T, J = T * (a.g.top_k + 1), nd = a.g.dim / 256, ni = a.g.I / 256;
   auto take = [&](size_t bytes) {
     uint8_t* r = p;
-    p += pf_round(bytes);
+    p += gx_round(bytes);
     return r;
   };
-  a.xh = (_Float16*)take((size_t)a.T * a.dim * 2);
-  a.xl = (_Float16*)take((size_t)a.T * a.dim * 2);
-  a.xsh = (_Float16*)take((size_t)a.T * nd * 16 * 2);
-  a.xsl = (_Float16*)take((size_t)a.T * nd * 16 * 2);
-  a.xinv = (float*)take((size_t)a.T * 4);
-  a.gsh = (float*)take((size_t)a.T * 4);
-  a.h = (float*)take(J * a.I * 4);
-  a.hh = (_Float16*)take(J * a.I * 2);
-  a.hl = (_Float16*)take(J * a.I * 2);
-  a.hsh = (_Float16*)take(J * ni * 16 * 2);
-  a.hsl = (_Float16*)take(J * ni * 16 * 2);
-  a.hinv = (float*)take(J * 4);
-  a.yk = (float*)take(J * a.dim * 4);
+  a.ximg = take(T * nd * GX_REC);
+  a.himg = take(J * ni * GX_REC);
+  a.g.h = (float*)take(J * a.g.I * 4);
+  a.g.yk = (float*)take(J * a.g.dim * 4);
+  a.g.gsh = (float*)take(T * 4);
   a.jobs = (int*)take(J * 4);
-  a.units = (int4*)p;
+  a.units = (int4*)take((1 + gx_max_groups(a.g.T, a.g.top_k, MOE_MAX_EXP, 32)) * 16);
+  return p;
 }
 
-// Activation rows per product tile from the expected jobs per routed expert.
-static int pf_mb(int T, int top_k, int n_exp) {
-  const double per = (double)T * top_k / n_exp;
-  return per >= 40 ? 4 : per >= 20 ? 2 : 1;
+size_t moe_prefill_work_bytes(int T, int dim, int I, int top_k) {
+  if (!gx_may_take(T, dim, I)) return 0;
+  T = std::min(T, MOE_PREFILL_MAX_TOKENS);
+  GxMoe a{};
+  a.g.T = T; a.g.dim = dim; a.g.I = I; a.g.top_k = top_k;
+  return (size_t)(gx_layout(a, nullptr) - (uint8_t*)nullptr);
 }
 
+// Expected jobs per routed expert from which groups hold up to 64 jobs instead
+// of 32: a group of 33..64 then costs one decode of the weights instead of two,
+// at two workgroups per CU instead of three.
+constexpr double MOE_GX_WIDE = 24;
+
+// The other paths' time grows with the jobs (chunks of two on the matrix cores
+// for Q4_K / Q6_K, one job at a time on the vector ALUs for the other kinds),
+// this one's mostly with the distinct experts, plus two more launches.  Times
+// in us, this path / the other, per layer with the router on MI355X.
 bool moe_prefill_takes(int T, int gu_kind, int down_kind, int dim, int I, int top_k, int n_exp) {
-  return T >= MOE_PREFILL_MIN_TOKENS && gu_kind == Q4_K && down_kind == Q6_K && dim % 256 == 0 && I % 256 == 0 &&
-         top_k >= 1 && top_k <= MOE_MAX_TOPK && n_exp >= 1 && n_exp <= MOE_MAX_EXP;
+  // The records are addressed with 32-bit offsets.
+  const size_t t = std::min(T, MOE_PREFILL_MAX_TOKENS);
+  if (!gx_may_take(T, dim, I) || gu_kind < 0 || gu_kind > Q8_0 || down_kind < 0 || down_kind > Q8_0 || top_k < 1 || top_k > MOE_MAX_TOPK || n_exp < 1 || n_exp > MOE_MAX_EXP ||
+      t * (top_k + 1) * (I / 256) * GX_REC >= (size_t)1 << 32 || t * (dim / 256) * GX_REC >= (size_t)1 << 32)
+    return false;
+  // Q4_K / Q6_K, 2048x768, 128 experts, top 8: 175 / 296 at 95 tokens.
+  if (T >= 96) return true;
+  const long jobs = (long)T * top_k;
+  // Q4_K / Q6_K: at 48 tokens 2048x768 with 128 experts, top 8 161 / 172; with
+  // 60, top 4 91 / 99; with 16, top 2 63 / 69 (at 32: 150 / 126, 90 / 77, 63 /
+  // 55).  Many jobs per expert pay earlier: 16 experts, top 8 61 / 67 at 16.
+  if (moe_mfma_kind(gu_kind) && moe_mfma_kind(down_kind)) return T >= 48 || (T >= 16 && jobs >= 6L * n_exp);
+  // Others: 128 experts, top 8 at 16 tokens Q5_K/Q6_K 122 / 139, Q2_K/Q3_K 103 /
+  // 110 (at 8: 96 / 90, 83 / 74); 16 experts, top 8 at 4 tokens Q5_K/Q6_K 54 / 66.
+  return T >= 16 || jobs >= 2L * n_exp;
 }
 
-hipError_t launch_moe_prefill(const MoeGroupedArgs& g, void* work, hipStream_t s) {
-  if (g.T < 1 || g.T > MOE_PREFILL_MAX_TOKENS) return hipErrorInvalidValue;
-  PfArgs a{};
-  a.gate = g.gate; a.up = g.up; a.down = g.down;
-  a.sh_gate = g.sh_gate; a.sh_up = g.sh_up; a.sh_down = g.sh_down;
-  a.gu_stride = g.gu_stride; a.d_stride = g.d_stride;
-  a.idx = g.idx; a.top_w = g.top_w; a.x = g.x; a.sgi = g.sgi; a.y = g.y;
-  a.T = g.T; a.top_k = g.top_k; a.n_exp = g.n_exp; a.dim = g.dim; a.I = g.I;
-  pf_bind(a, work);
-  const int J = a.T * (a.top_k + 1);
-  const int mb = pf_mb(a.T, a.top_k, a.n_exp), bp = 16 * mb;
-  const size_t groups = pf_max_groups(a.T, a.top_k, a.n_exp, bp);
-  hipError_t e = launch_xsplit(32, a.x, a.T, a.T, a.dim, a.xh, a.xl, a.xsh, a.xsl, a.xinv, s);
-  if (e != hipSuccess) return e;
-  switch (mb) {
-    case 1: hipLaunchKernelGGL(moe_pf_plan<16>, dim3(1), dim3(1024), 0, s, a); break;
-    case 2: hipLaunchKernelGGL(moe_pf_plan<32>, dim3(1), dim3(1024), 0, s, a); break;
-    default: hipLaunchKernelGGL(moe_pf_plan<64>, dim3(1), dim3(1024), 0, s, a); break;
+template <int KIND, int NVM, bool DOWN>
+static hipError_t gx_expert(const GxMoe& a, size_t groups, int bp, int tiles, hipStream_t s) {
+  const int shared = (a.g.T + bp - 1) / bp * tiles;
+  const size_t units = std::max(groups * tiles, (size_t)shared);
+  const size_t grid = (size_t)((shared + 7) & ~7) + (units - shared + 7) / 8 * 8;
+  constexpr int lds = GxLds<KIND, NVM>::BYTES;
+  // More than 64 KB of LDS has to be asked for.
+  if (lds > 60 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(moe_gx_expert<KIND, NVM, DOWN>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return e;
   }
-  const dim3 gu((unsigned)(groups * (a.I / 64))), dn((unsigned)(groups * (a.dim / 64)));
-  const bool wide = a.I / 256 <= PF_DN_COLS;
-  const dim3 dnw((unsigned)(groups * ((a.dim / 64 + PF_DN_TILES - 1) / PF_DN_TILES)));
-  switch (mb) {
-    case 1: hipLaunchKernelGGL(moe_pf_gate_up<1>, gu, dim3(256), 0, s, a); break;
-    case 2: hipLaunchKernelGGL(moe_pf_gate_up<2>, gu, dim3(256), 0, s, a); break;
-    default: hipLaunchKernelGGL(moe_pf_gate_up<4>, gu, dim3(256), 0, s, a); break;
-  }
-  e = launch_xsplit(16, a.h, J, J, a.I, a.hh, a.hl, a.hsh, a.hsl, a.hinv, s);
-  if (e != hipSuccess) return e;
-  if (wide) {
-    switch (mb) {
-      case 1: hipLaunchKernelGGL((moe_pf_down_wide<1, 16>), dnw, dim3(256), 0, s, a); break;
-      case 2: hipLaunchKernelGGL((moe_pf_down_wide<2, 32>), dnw, dim3(256), 0, s, a); break;
-      default: hipLaunchKernelGGL((moe_pf_down_wide<2, 64>), dnw, dim3(256), 0, s, a); break;
-    }
-  } else {
-    switch (mb) {
-      case 1: hipLaunchKernelGGL((moe_pf_down<1, 16>), dn, dim3(256), 0, s, a); break;
-      case 2: hipLaunchKernelGGL((moe_pf_down<2, 32>), dn, dim3(256), 0, s, a); break;
-      default: hipLaunchKernelGGL((moe_pf_down<2, 64>), dn, dim3(256), 0, s, a); break;
-    }
-  }
-  hipLaunchKernelGGL(moe_pf_gates, dim3((a.T + 3) / 4), dim3(256), 0, s, a);
-  hipLaunchKernelGGL(moe_pf_combine, dim3((a.dim + 255) / 256, a.T), dim3(256), 0, s, a);
+  hipLaunchKernelGGL((moe_gx_expert<KIND, NVM, DOWN>), dim3((unsigned)grid), dim3(256), lds, s, a, tiles, shared);
   return hipGetLastError();
+}
+
+template <bool DOWN>
+static hipError_t gx_experts(const GxMoe& a, int kind, size_t groups, int bp, int tiles, hipStream_t s) {
+#define KQ_GX(K) \
+  case K: return bp == 64 ? gx_expert<K, 2, DOWN>(a, groups, bp, tiles, s) : gx_expert<K, 1, DOWN>(a, groups, bp, tiles, s);
+  switch (kind) {
+    KQ_GX(Q4_K) KQ_GX(Q6_K) KQ_GX(Q5_K) KQ_GX(Q3_K) KQ_GX(Q2_K) KQ_GX(Q8_0)
+    default: return hipErrorInvalidValue;
+  }
+#undef KQ_GX
+}
+
+hipError_t launch_moe_prefill(const MoeGroupedArgs& g, int gu_kind, int down_kind, void* work, hipStream_t s) {
+  if (g.T < 1 || g.T > MOE_PREFILL_MAX_TOKENS) return hipErrorInvalidValue;
+  GxMoe a{};
+  a.g = g;
+  gx_layout(a, (uint8_t*)work);
+  const int J = g.T * (g.top_k + 1), nd = g.dim / 256, ni = g.I / 256;
+  const int bp = (double)g.T * g.top_k / g.n_exp > MOE_GX_WIDE ? 64 : 32;
+  const size_t groups = gx_max_groups(g.T, g.top_k, g.n_exp, bp);
+  const int split = (g.T * nd * 8 + PREP_THREADS - 1) / PREP_THREADS;
+  const dim3 prep(1 + split + (g.T + PREP_THREADS / 64 - 1) / (PREP_THREADS / 64));
+  switch (gx_sums(gu_kind)) {
+    case 0: hipLaunchKernelGGL(moe_gx_prep<0>, prep, dim3(PREP_THREADS), 0, s, a, bp, split); break;
+    case 1: hipLaunchKernelGGL(moe_gx_prep<1>, prep, dim3(PREP_THREADS), 0, s, a, bp, split); break;
+    default: hipLaunchKernelGGL(moe_gx_prep<2>, prep, dim3(PREP_THREADS), 0, s, a, bp, split); break;
+  }
+  hipError_t e = gx_experts<false>(a, gu_kind, groups, bp, g.I / 64, s);
+  if (e != hipSuccess) return e;
+  const dim3 hs((J * ni + 31) / 32);
+  switch (gx_sums(down_kind)) {
+    case 0: hipLaunchKernelGGL(moe_gx_hsplit<0>, hs, dim3(256), 0, s, a, J); break;
+    case 1: hipLaunchKernelGGL(moe_gx_hsplit<1>, hs, dim3(256), 0, s, a, J); break;
+    default: hipLaunchKernelGGL(moe_gx_hsplit<2>, hs, dim3(256), 0, s, a, J); break;
+  }
+  e = gx_experts<true>(a, down_kind, groups, bp, g.dim / 128, s);
+  if (e != hipSuccess) return e;
+  return launch_moe_combine(a.g, s);
 }
 
 }  // namespace kq

@@ -248,6 +248,7 @@ __global__ __launch_bounds__(64 * NW) void kq_mv_mfma16n(const uint8_t* __restri
 static thread_local int g_engine = 0;
 
 void set_matvec_engine(int engine) { g_engine = engine; }
+int matvec_engine() { return g_engine; }
 
 bool matvec_mfma_takes(int kind) {
   return (kind == Q4_K || kind == Q6_K || kind == Q2_K || kind == Q5_K || kind == Q3_K) && g_engine == 0;
