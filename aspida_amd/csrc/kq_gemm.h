@@ -332,13 +332,16 @@ __device__ __forceinline__ void gx_split(const float* x, int u, F&& frag, G&& su
   for (int i = 0; i < 8; ++i) a = fmaxf(a, fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w))));
 #pragma unroll
   for (int o = 1; o < 8; o <<= 1) a = fmaxf(a, __shfl_xor(a, o, 64));
-  // S = 2^(14 - e) with a < 2^e, at most 2^116; 1 for zero or non-finite columns.
+  // S = 2^(14 - e) with a < 2^e, at most 2^116; 1 for a column of zeros.  Beside
+  // an Inf 2^-114, at which no finite element becomes one too.
   int e = 0;
-  const bool scaled = a > 0.f && __builtin_isfinite(a);
-  if (scaled) (void)frexpf(a, &e);
-  const int ex = scaled ? min(14 - e, 116) : 0;
+  const bool inf = __builtin_isinf(a);
+  if (a > 0.f && !inf) (void)frexpf(a, &e);
+  const int ex = inf ? -114 : a > 0.f ? min(14 - e, 116) : 0;
   const float S = ldexpf(1.f, ex);
   if (u == 0) *reinterpret_cast<float*>(inv) = ldexpf(1.f, -ex);
+  // What hi leaves, at most 8; the clamp takes Inf - Inf, so that an Inf stays one.
+  auto rest = [](float x, _Float16 hi) { return (_Float16)__builtin_amdgcn_fmed3f(x - (float)hi, -32.f, 32.f); };
   float part[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -350,9 +353,8 @@ __device__ __forceinline__ void gx_split(const float* x, int u, F&& frag, G&& su
       x1.x *= S; x1.y *= S; x1.z *= S; x1.w *= S;
       const h8 hi = {(_Float16)x0.x, (_Float16)x0.z, (_Float16)x0.y, (_Float16)x0.w,
                      (_Float16)x1.x, (_Float16)x1.z, (_Float16)x1.y, (_Float16)x1.w};
-      const h8 lo = {(_Float16)(x0.x - (float)hi[0]), (_Float16)(x0.z - (float)hi[1]), (_Float16)(x0.y - (float)hi[2]),
-                     (_Float16)(x0.w - (float)hi[3]), (_Float16)(x1.x - (float)hi[4]), (_Float16)(x1.z - (float)hi[5]),
-                     (_Float16)(x1.y - (float)hi[6]), (_Float16)(x1.w - (float)hi[7])};
+      const h8 lo = {rest(x0.x, hi[0]), rest(x0.z, hi[1]), rest(x0.y, hi[2]), rest(x0.w, hi[3]),
+                     rest(x1.x, hi[4]), rest(x1.z, hi[5]), rest(x1.y, hi[6]), rest(x1.w, hi[7])};
       *reinterpret_cast<h8*>(frag(4 * u + 2 * b, h)) = hi;
       *reinterpret_cast<h8*>(frag(4 * u + 2 * b + 1, h)) = lo;
       q[2 * b] = (x0.x + x0.y) + (x0.z + x0.w);

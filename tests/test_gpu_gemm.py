@@ -102,6 +102,23 @@ def test_gemm_non_finite_vector_stays_its_own(kind):
     assert not np.any(np.isfinite(Y[3]))
 
 
+@pytest.mark.parametrize("kind", [aa.Q3_K, aa.Q8_0], ids=lambda k: aa.KIND_NAMES[k])
+def test_gemm_infinite_activation(kind):
+    """An Inf beside finite elements as large as f32 holds gives the weight's
+    sign times Inf, as one f32 sum does (NaN where the weight is 0).  The kinds
+    without a min term, whose weight enters as one exact factor."""
+    batch, out_dim, in_dim = 40, 96, 768
+    gen = synth.rng(4500 + kind)
+    w = synth.weight_np(kind, out_dim, in_dim, gen)
+    X = synth.activations_np(batch * in_dim, gen).reshape(batch, in_dim)
+    X[3, 300], X[35, 511], X[35, 400] = np.inf, -np.inf, 3e38
+    Y = _run(kind, w, X, in_dim, out_dim)
+    W = oracle.dequant(kind, w, in_dim, out_dim).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        assert np.array_equal(Y[3], (np.inf * W[:, 300]).astype(np.float32), equal_nan=True)
+        assert np.array_equal(Y[35], (-np.inf * W[:, 511]).astype(np.float32), equal_nan=True)
+
+
 def test_gemm_replays_in_a_graph():
     """A captured product (columns split, counters re-armed in the kernel)
     replayed with eager products of another shape between the replays."""
