@@ -253,9 +253,9 @@ size_t mm_work_bytes(int in_dim, int out_dim, int batch) {
     if (bp >= batch) break;
   }
   if (in_dim % 1024 == 0) n = std::max(n, kq::mmw_workspace_bytes(in_dim, out_dim, std::min(batch, 64)));
-  // From 64 vectors on, room for any batch, so that a stream warmed up with 64
-  // may capture larger products.
-  n = std::max(n, kq::gemm_workspace_bytes(in_dim, out_dim, batch >= 64 ? kq::GEMM_STEP : batch));
+  // Room for any batch, so that a stream warmed up with a small one may capture
+  // larger products.
+  n = std::max(n, kq::gemm_workspace_bytes(in_dim, out_dim, kq::GEMM_STEP));
   return n;
 }
 

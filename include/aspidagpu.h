@@ -157,7 +157,7 @@ int aspida_kq_matvec2_packed_dev(int kind_a, const void *packed_a, int out_a, fl
  * which run on the vector kernel, each row bit-identical to
  * aspida_kq_matvec_packed_dev on it under aspida_kq_set_mv_engine(1).
  * x must be 16-byte aligned; workspace as for aspida_kq_matvec_packed_dev
- * (sized by in_dim, out_dim and the batch; from 64 vectors on for any batch).
+ * (sized by in_dim and out_dim, the many-vector part for any batch).
  * The same math as the reference's batched kernels (gpu/gpu_matvec.cu:234-382)
  * without its batch limit of 32. */
 int aspida_kq_matmul_packed_dev(int kind, const void *packed, int in_dim, int out_dim, int batch,

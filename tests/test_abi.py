@@ -183,6 +183,18 @@ def test_matmul_workspace_covers_every_launch(lib):
                 assert alloc >= need, (aa.KIND_NAMES[kind], in_dim, out_dim, batch, alloc, need)
 
 
+@pytest.mark.parametrize("kind", aa.KINDS)
+def test_matmul_workspace_of_two_vectors_holds_any_batch(lib, kind):
+    """A stream warmed up with two vectors may capture a product of any number
+    of vectors on the same matrix where the many-vector kernel takes it (Q5_K,
+    Q3_K, Q2_K and Q8_0: always; Q4_K and Q6_K: above 64)."""
+    every = kind not in (aa.Q4_K, aa.Q6_K)
+    for in_dim, out_dim in [(256, 64), (768, 2048), (4096, 4096), (4096, 28672), (14336, 4096), (14336, 1024)]:
+        alloc, _ = _matmul_ws(lib, kind, in_dim, out_dim, 2)
+        for batch in ([4, 8, 16, 32, 33, 64] if every else []) + [65, 96, 128, 511, 512, 513, 576, 1024]:
+            assert alloc >= _matmul_ws(lib, kind, in_dim, out_dim, batch)[1], (in_dim, out_dim, batch)
+
+
 def test_matmul_workspace_advisor_shapes(lib):
     """The shapes where a 64-row padding undersized the buffer: Q6_K
     8960->1536 at B=48 and Q4_K/Q6_K 3584x3584 at B=48 and 65 -- on the
