@@ -30,11 +30,6 @@ __device__ __forceinline__ uint32_t pack_h(_Float16 a, _Float16 b) {
   return (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
 }
 
-// The split of B rows of in_dim activations, one workgroup per row
-// (kq_mmq.hip); rows b with B <= b < grid rows are written as zeros.
-hipError_t launch_xsplit(int sub, const float* X, int B, int grid_rows, int in_dim, _Float16* xh, _Float16* xl,
-                         _Float16* sh, _Float16* sl, float* inv, hipStream_t s);
-
 // ---- shared pieces ---------------------------------------------------------
 
 __device__ __forceinline__ h8 as_h8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {

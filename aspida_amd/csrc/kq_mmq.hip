@@ -92,15 +92,6 @@ __global__ __launch_bounds__(1024) void kq_xsplit(const float* __restrict__ X, i
   }
 }
 
-hipError_t launch_xsplit(int sub, const float* X, int B, int grid_rows, int in_dim, _Float16* xh, _Float16* xl,
-                         _Float16* sh, _Float16* sl, float* inv, hipStream_t s) {
-  if (sub == 32)
-    hipLaunchKernelGGL(kq_xsplit<32>, dim3(grid_rows), dim3(1024), 0, s, X, B, in_dim, xh, xl, sh, sl, inv);
-  else
-    hipLaunchKernelGGL(kq_xsplit<16>, dim3(grid_rows), dim3(1024), 0, s, X, B, in_dim, xh, xl, sh, sl, inv);
-  return hipGetLastError();
-}
-
 struct MmArgs {
   const uint8_t* P;   // packed weights
   int nsb, out_dim, B, spw;
