@@ -2,7 +2,7 @@
 // packed weights of every kind on the matrix cores: Y[b][out] = W X[b].
 //
 //   kq_gx_split   X as f16 hi / lo fragments per 32 vectors and column
-//                 (kq_gemm.h), one workgroup each
+//                 (kq_gemm.h), four workgroups each
 //   kq_gemm       a workgroup of four waves per 128 rows x 32 or 64 vectors x a
 //                 run of columns, each wave its own 32 rows: weights decoded in
 //                 registers, activations shared through LDS;
@@ -25,15 +25,14 @@
 
 namespace kq {
 
-
-// One thread per 32 elements of one of 32 vectors.
+// 32 threads per vector, eight of a block's 32 vectors per workgroup.
 template <int SUMS>
 __global__ __launch_bounds__(256) void kq_gx_split(const float* __restrict__ X, int B, int in_dim,
                                                    uint8_t* __restrict__ img) {
-  const int m = threadIdx.x >> 3, u = threadIdx.x & 7, nsb = in_dim / 256;
+  const int m = 8 * blockIdx.z + (threadIdx.x >> 5), t = threadIdx.x & 31, nsb = in_dim / 256;
   const int s = blockIdx.x, row = blockIdx.y * 32 + m;
   uint8_t* out = img + ((size_t)blockIdx.y * nsb + s) * GX_COL;
-  gx_split<SUMS>(row < B ? X + (size_t)row * in_dim + 256 * s : nullptr, u,
+  gx_split<SUMS>(row < B ? X + (size_t)row * in_dim + 256 * s : nullptr, t,
                  [&](int f, int h) { return out + f * 1024 + (h * 32 + m) * 16; },
                  [&](int i, int h) { return out + GX_SUM + i * 1024 + (h * 32 + m) * 16; }, out + GX_AUX + 4 * m);
 }
@@ -255,7 +254,7 @@ hipError_t launch_gemm(int kind, const void* P, int in_dim, int out_dim, int bat
   a.part = (float*)((uint8_t*)work + gemm_image_bytes(in_dim, batch));
   a.Y = Y;
   a.count = count;
-  const dim3 gs((unsigned)a.nsb, (unsigned)a.vblocks);
+  const dim3 gs((unsigned)a.nsb, (unsigned)a.vblocks, 4);
   switch (gx_sums(kind)) {
     case 0: hipLaunchKernelGGL(kq_gx_split<0>, gs, dim3(256), 0, s, X, batch, in_dim, (uint8_t*)work); break;
     case 1: hipLaunchKernelGGL(kq_gx_split<1>, gs, dim3(256), 0, s, X, batch, in_dim, (uint8_t*)work); break;

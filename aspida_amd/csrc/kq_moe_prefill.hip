@@ -27,10 +27,10 @@
 // Bound by the matrix cores and the vector instructions around them (kq_gemm.h)
 // from about 100 tokens, by the weights' latency below.  The Qwen3-MoE layer
 // (2048x768, 128 experts and a shared one, top 8, Q4_K / Q6_K, router included):
-// 1024 tokens 436 us (889 on 16x16x16 products of 64-job tiles), 512 283 (474),
+// 1024 tokens 429 us (889 on 16x16x16 products of 64-job tiles), 512 283 (474),
 // 256 200 (352), 128 184 (265), 64 166 (216); Q5_K / Q6_K 256 tokens 205 (1468
-// on the vector ALUs).  At 1024: prep 14, gate/up 234, h split 20, down 156,
-// combine 22.
+// on the vector ALUs).  At 1024: router 30, prep 12, gate/up 236, h split 14,
+// down 155, combine 22.
 #include <math.h>
 
 #include <algorithm>
@@ -103,10 +103,10 @@ __device__ __forceinline__ void gx_plan(const GxMoe& a, int BP) {
   if (tid == 0) a.units[0] = make_int4(groups, 0, 0, 0);
 }
 
-// Thread u of row `row`, column s of a record image.
+// Thread t (0..31) of one record.
 template <int SUMS>
-__device__ __forceinline__ void gx_record(const float* x, uint8_t* rec, int u) {
-  gx_split<SUMS>(x, u, [&](int f, int h) { return rec + f * 32 + h * 16; },
+__device__ __forceinline__ void gx_record(const float* x, uint8_t* rec, int t) {
+  gx_split<SUMS>(x, t, [&](int f, int h) { return rec + f * 32 + h * 16; },
                  [&](int i, int h) { return rec + GX_RAUX + i * 32 + h * 16; }, rec + GX_RINV);
 }
 
@@ -120,9 +120,9 @@ __global__ __launch_bounds__(PREP_THREADS) void moe_gx_prep(GxMoe a, int BP, int
   }
   const int T = a.g.T, nd = a.g.dim / 256, b = blockIdx.x - 1;
   if (b < split_blocks) {
-    const int q = b * (PREP_THREADS / 8) + (threadIdx.x >> 3), row = q / nd, s = q % nd;
+    const int q = b * (PREP_THREADS / 32) + (threadIdx.x >> 5), row = q / nd, s = q % nd;
     if (row < T)
-      gx_record<SUMS>(a.g.x + (size_t)row * a.g.dim + 256 * s, a.ximg + (size_t)q * GX_REC, threadIdx.x & 7);
+      gx_record<SUMS>(a.g.x + (size_t)row * a.g.dim + 256 * s, a.ximg + (size_t)q * GX_REC, threadIdx.x & 31);
     return;
   }
   const int t = (b - split_blocks) * (PREP_THREADS / 64) + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -145,8 +145,8 @@ __global__ __launch_bounds__(PREP_THREADS) void moe_gx_prep(GxMoe a, int BP, int
 
 template <int SUMS>
 __global__ __launch_bounds__(256) void moe_gx_hsplit(GxMoe a, int rows) {
-  const int ni = a.g.I / 256, q = blockIdx.x * 32 + (threadIdx.x >> 3), row = q / ni, s = q % ni;
-  if (row < rows) gx_record<SUMS>(a.g.h + (size_t)row * a.g.I + 256 * s, a.himg + (size_t)q * GX_REC, threadIdx.x & 7);
+  const int ni = a.g.I / 256, q = blockIdx.x * 8 + (threadIdx.x >> 5), row = q / ni, s = q % ni;
+  if (row < rows) gx_record<SUMS>(a.g.h + (size_t)row * a.g.I + 256 * s, a.himg + (size_t)q * GX_REC, threadIdx.x & 31);
 }
 
 // The unit of workgroup b among N (groups times tiles): the shared expert's S
@@ -352,7 +352,7 @@ hipError_t launch_moe_prefill(const MoeGroupedArgs& g, int gu_kind, int down_kin
   const int J = g.T * (g.top_k + 1), nd = g.dim / 256, ni = g.I / 256;
   const int bp = (double)g.T * g.top_k / g.n_exp > MOE_GX_WIDE ? 64 : 32;
   const size_t groups = gx_max_groups(g.T, g.top_k, g.n_exp, bp);
-  const int split = (g.T * nd * 8 + PREP_THREADS - 1) / PREP_THREADS;
+  const int split = (g.T * nd * 32 + PREP_THREADS - 1) / PREP_THREADS;
   const dim3 prep(1 + split + (g.T + PREP_THREADS / 64 - 1) / (PREP_THREADS / 64));
   switch (gx_sums(gu_kind)) {
     case 0: hipLaunchKernelGGL(moe_gx_prep<0>, prep, dim3(PREP_THREADS), 0, s, a, bp, split); break;
@@ -361,7 +361,7 @@ hipError_t launch_moe_prefill(const MoeGroupedArgs& g, int gu_kind, int down_kin
   }
   hipError_t e = gx_experts<false>(a, gu_kind, groups, bp, g.I / 64, s);
   if (e != hipSuccess) return e;
-  const dim3 hs((J * ni + 31) / 32);
+  const dim3 hs((J * ni + 7) / 8);
   switch (gx_sums(down_kind)) {
     case 0: hipLaunchKernelGGL(moe_gx_hsplit<0>, hs, dim3(256), 0, s, a, J); break;
     case 1: hipLaunchKernelGGL(moe_gx_hsplit<1>, hs, dim3(256), 0, s, a, J); break;
