@@ -169,6 +169,8 @@ size_t gemm_workspace_bytes(int in_dim, int out_dim, int batch) {
 // MI355X with every launch of a product counted.
 bool gemm_takes(int kind, int in_dim, int out_dim, int batch) {
   const int nsb = in_dim / 256, tiles = (out_dim + 63) / 64;
+  // Offsets within a vector block's image are 31 bits.
+  if (nsb > INT32_MAX / GX_COL) return false;
   const long units = (long)nsb * tiles;
   // Below 192 tiles (3/4 of a 256-CU device) the one-pass kernel takes 16-row
   // blocks and converts the activations once per 16 rows instead of per 64.

@@ -195,6 +195,14 @@ def test_matmul_workspace_of_two_vectors_holds_any_batch(lib, kind):
             assert alloc >= _matmul_ws(lib, kind, in_dim, out_dim, batch)[1], (in_dim, out_dim, batch)
 
 
+def test_matmul_of_very_long_rows_keeps_the_vector_kernel(lib):
+    """Rows whose activation image passes 2 GB per 32 vectors (58254 columns)
+    stay on the vector kernel, which needs no workspace."""
+    longest = ((1 << 31) - 1) // (36 * 1024)
+    assert _matmul_ws(lib, aa.Q5_K, 256 * longest, 64, 16)[1] > 0
+    assert _matmul_ws(lib, aa.Q5_K, 256 * (longest + 1), 64, 16)[1] == 0
+
+
 def test_matmul_workspace_advisor_shapes(lib):
     """The shapes where a 64-row padding undersized the buffer: Q6_K
     8960->1536 at B=48 and Q4_K/Q6_K 3584x3584 at B=48 and 65 -- on the
