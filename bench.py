@@ -96,7 +96,7 @@ def size_sweep_table(torch, aa, synth, seed, stream):
 
 # Launches of one layer: q|k and v share their input and run as one launch.
 LAYER_LAUNCHES = [("qk", "v"), ("o",), ("gate_up",), ("down",)]
-# Token counts of the MoE prefill rows (the grouped-GEMM path from 96 tokens).
+# Token counts of the MoE prefill rows (the grouped many-job products).
 PREFILL_TOKENS = (128, 256, 512, 1024)
 
 
