@@ -409,7 +409,7 @@ def gemm_takes(aa, kind, inp, out, B):
         if B > 32:
             return nsb >= 16
         if B > 16:
-            return nsb >= 32 or units >= 3584
+            return nsb >= 16 or units >= 3584
         return B > 4 and narrow and (units >= (2048 if B > 8 else 3584) or nsb >= 48)
     if B > 32:
         return B > 48 or units > 1024 or nsb < 32
