@@ -31,6 +31,9 @@
 // 2.8e-7 for a sequential f32 sum; the split itself 4.4e-8).  Columns are
 // added in groups of GX_GROUP, groups then among each other.
 #pragma once
+#include <type_traits>
+
+#include "kq_gx_stages.h"
 #include "kq_mmq.h"
 
 namespace kq {
@@ -45,9 +48,6 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 constexpr int GX_AUX = 32 * 1024;
 constexpr int GX_SUM = GX_AUX + 1024;
 constexpr int GX_COL = 36 * 1024;
-// 64-element stages (8 KB per vector block) in LDS: as many as leave room for
-// three workgroups per CU (NV = 1) or two (NV = 2).
-constexpr int gx_ring(int nv) { return nv == 1 ? 6 : 4; }
 constexpr int GX_STAGE = 8 * 1024;
 constexpr int GX_GROUP = 8;
 
@@ -401,6 +401,16 @@ template <int N>
 __device__ __forceinline__ void gx_wait_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
+// The one before stage j (a constant once its loop is unrolled).
+template <int KIND, int NV, bool LAST>
+__device__ __forceinline__ void gx_stage_barrier(int j) {
+  switch (j) {
+    case 0: gx_wait_barrier<gx_stage_wait(KIND, NV, 0, LAST)>(); break;
+    case 1: gx_wait_barrier<gx_stage_wait(KIND, NV, 1, LAST)>(); break;
+    case 2: gx_wait_barrier<gx_stage_wait(KIND, NV, 2, LAST)>(); break;
+    default: gx_wait_barrier<gx_stage_wait(KIND, NV, 3, LAST)>(); break;
+  }
+}
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p;
 }
@@ -467,11 +477,6 @@ __device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, i
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t ring = __builtin_amdgcn_readfirstlane(lds_offset(lds)), lo16 = 16 * lane;
   constexpr int R = gx_ring(NV);
-  // Loads a wave issues per R - 2 consecutive stages: the fragments, and the
-  // body loads (one per stage, two for Q8_0, three in every other one for Q6_K,
-  // one in every other one for Q2_K and Q3_K).
-  constexpr int DMA = (R - 2) * 2 * NV;
-  constexpr int BODY = (R - 2) * (KIND == Q8_0 ? 4 : KIND == Q6_K ? 3 : KIND == Q2_K || KIND == Q3_K ? 1 : 2) / 2;
   const int last = 4 * (s1 - s0) - 1;  // stages
   // Stage g's 8 NV fragments, 2 NV per wave (past the end the last stage
   // again, into a slot nobody reads, so that every stage issues as many).
@@ -486,7 +491,7 @@ __device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, i
     }
   };
   auto dma_aux = [&](int c) {  // of column s0 + c, one fragment per wave in turn
-    const int s = min(s0 + c, s1 - 1);
+    const int s = s0 + c;
     const uint32_t dst = ring + L::AUX0 + (c & 1) * NV * L::AUXB;
 #pragma unroll
     for (int v = 0; v < NV; ++v)
@@ -512,11 +517,15 @@ __device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, i
   f16v sum[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) sum[v] = acc[v] = zero16();
-  for (int s = s0; s < s1; ++s) {
-    const int c = s - s0;
-    if (s + 1 < s1) g0 += GB;
+  // One column; the last one, a form of its own, has no next one's weights to
+  // load.
+  auto column = [&](const int c, auto is_last) {
+    constexpr bool LAST = decltype(is_last)::value;
     wt.next_head();
-    wt.load_head(g0, row, ro, h);
+    if constexpr (!LAST) {
+      g0 += GB;
+      wt.load_head(g0, row, ro, h);
+    }
     const auto sc = wt.scales();
     f16v th[NV], tl[NV];
 #pragma unroll
@@ -524,10 +533,9 @@ __device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, i
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int g = 4 * c + j;
-      // This wave's loads of stage g are done (the R - 2 stages issued after it
-      // count DMA + BODY later ones) and its reads of stage g - 1; then
-      // everyone's.
-      gx_wait_barrier<DMA + BODY>();
+      // This wave's loads of stage g are done and its reads of stage g - 1;
+      // then everyone's.
+      gx_stage_barrier<KIND, NV, LAST>(j);
       const uint8_t* st = lds + slot * NV * GX_STAGE + lo16;
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
@@ -573,8 +581,8 @@ __device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, i
           }
         }
       }
-      wt.load_body(g0, ro, h, j);
-      if (j == 1) dma_aux(c + 1);
+      if constexpr (!LAST) wt.load_body(g0, ro, h, j);
+      if (!LAST && j == 1) dma_aux(c + 1);
       dma_stage(g + R - 1, fill);
       slot = slot + 1 == R ? 0 : slot + 1;
       fill = fill + 1 == R ? 0 : fill + 1;
@@ -613,7 +621,9 @@ __device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, i
         acc[v] = zero16();
       }
     }
-  }
+  };
+  for (int c = 0; c < s1 - s0 - 1; ++c) column(c, std::false_type{});
+  column(s1 - s0 - 1, std::true_type{});
 #pragma unroll
   for (int v = 0; v < NV; ++v) acc[v] += sum[v];
   // No load may reach LDS after the workgroup has ended.

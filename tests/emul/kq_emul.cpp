@@ -36,6 +36,7 @@ using std::max;
 using std::min;
 
 #include "../../aspida_amd/csrc/kq_blocks.h"
+#include "../../aspida_amd/csrc/kq_gx_stages.h"
 #include "../../aspida_amd/csrc/kq_packed.h"
 
 extern "C" float kq_emul_quarter(int kind, const uint8_t* sb, int c, const float* xs, const float* xq) {
@@ -93,3 +94,8 @@ extern "C" float kq_emul_packed_row(int kind, const uint8_t* g, int lane, const 
   }
   return NAN;
 }
+
+// The many-vector core's load stages (kq_gx_stages.h).
+extern "C" int kq_emul_gx_ring(int nv) { return kq::gx_ring(nv); }
+extern "C" int kq_emul_gx_body_loads(int kind, int j) { return kq::gx_body_loads(kind, j); }
+extern "C" int kq_emul_gx_stage_wait(int kind, int nv, int j, int last) { return kq::gx_stage_wait(kind, nv, j, last != 0); }
