@@ -28,8 +28,14 @@
 // matrix cores round each 16-element step to f32 at the size of the running
 // sum, so one chain taking both rounds twice as often (measured against 64
 // bits over 256 elements: 1.5e-7 with hi and lo alternating, 1.07e-7 apart,
-// 2.8e-7 for a sequential f32 sum; the split itself 4.4e-8).  Columns are
-// added in groups of GX_GROUP, groups then among each other.
+// 2.8e-7 for a sequential f32 sum; the split itself 4.4e-8).  Q5_K and Q2_K,
+// whose code and min sums cancel most, have two chains of hi, one per half
+// column (gx_halves); Q2_K's min sums, whose mins are as large as its codes,
+// have three planes and are those of the split's own values.  Error over f64,
+// without / with both / of the f32 vector kernel: Q5_K 4096x1024 x 16 1.31e-7 /
+// 1.07e-7 / 1.25e-7, Q2_K 9.7e-8 / 8.8e-8 / 1.07e-7, with one activation of 1e4
+// in 1024 Q5_K 1.37e-7 / 9.4e-8 / 1.48e-7, Q2_K 1.65e-7 / 1.20e-7 / 1.03e-7.
+// Columns are added in groups of GX_GROUP, groups then among each other.
 #pragma once
 #include <type_traits>
 
@@ -44,7 +50,7 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 // of 1 KB (step ks, plane p at (2 ks + p) KB; lane l's eight halves at 16 l),
 // at GX_AUX 1 / S of the 32 vectors (f32) and from GX_SUM the min-term
 // fragments (sums of 32: one, hi in the lower lane half and lo in the upper;
-// sums of 16: two, hi and lo).
+// sums of 16: three, hi, what it leaves as lo, and what both leave).
 constexpr int GX_AUX = 32 * 1024;
 constexpr int GX_SUM = GX_AUX + 1024;
 constexpr int GX_COL = 36 * 1024;
@@ -53,6 +59,10 @@ constexpr int GX_GROUP = 8;
 
 // Which sums the kind's min term takes: 0 none, 1 sums of 32, 2 sums of 16.
 __host__ __device__ constexpr int gx_sums(int kind) { return kind == Q4_K || kind == Q5_K ? 1 : kind == Q2_K ? 2 : 0; }
+// Their fragments.
+__host__ __device__ constexpr int gx_sum_frags(int sums) { return sums == 2 ? 3 : sums; }
+// Whether hi of a column's first half has a chain of its own.
+__host__ __device__ constexpr bool gx_halves(int kind) { return kind == Q5_K || kind == Q2_K; }
 
 __device__ __forceinline__ f16v mfma3216(h8 a, h8 b, f16v c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
@@ -363,6 +373,12 @@ __device__ __forceinline__ void gx_split(const float* x, int t, F&& frag, G&& su
     *reinterpret_cast<_Float16*>(sums(i, half) + 2 * p) = (_Float16)y;
   };
   if constexpr (SUMS != 0) {
+    if constexpr (SUMS == 2) {  // of what hi and lo hold, so that code and min terms cancel on the same values
+      x0 = make_float4((float)hi[0] + (float)lo[0], (float)hi[2] + (float)lo[2], (float)hi[1] + (float)lo[1],
+                       (float)hi[3] + (float)lo[3]);
+      x1 = make_float4((float)hi[4] + (float)lo[4], (float)hi[6] + (float)lo[6], (float)hi[5] + (float)lo[5],
+                       (float)hi[7] + (float)lo[7]);
+    }
     float y = ((x0.x + x0.y) + (x0.z + x0.w)) + ((x1.x + x1.y) + (x1.z + x1.w));
     y += __shfl_xor(y, 1, 64);
     if constexpr (SUMS == 1) y += __shfl_xor(y, 2, 64);
@@ -372,7 +388,9 @@ __device__ __forceinline__ void gx_split(const float* x, int t, F&& frag, G&& su
       if (b == 0) put(u, 0, h, h ? y - yh : yh);
     } else {
       const int c = 2 * u + h;
-      put(c & 7, b, c >> 3, b ? y - yh : yh);
+      const float yl = (float)(_Float16)(y - yh);
+      put(c & 7, b, c >> 3, b ? yl : yh);
+      if (b) put(c & 7, 2, c >> 3, (y - yh) - yl);
     }
   }
 }
@@ -426,7 +444,8 @@ template <int NV> struct GxDense {
     gx_dma16(img[v], lo16, s * GX_COL + f * 1024, dst);
   }
   __device__ __forceinline__ void aux(int v, int s, int i, uint32_t dst) const {
-    gx_dma16(img[v], lo16, s * GX_COL + GX_AUX + 1024 * i, dst);
+    if (i == 0) gx_dma4(img[v], lo16 >> 2, s * GX_COL + GX_AUX, dst);
+    else gx_dma16(img[v], lo16, s * GX_COL + GX_SUM + 1024 * (i - 1), dst);
   }
 };
 
@@ -434,7 +453,7 @@ template <int NV> struct GxDense {
 // record (row, column) holds the 32 fragments' 2 x 16 bytes of its vector (32 f
 // + 16 h), at GX_RAUX the sums in fragment order and at GX_RINV 1 / S.
 constexpr int GX_RAUX = 1024;
-constexpr int GX_RINV = GX_RAUX + 64;
+constexpr int GX_RINV = GX_RAUX + 96;
 constexpr int GX_REC = 1152;
 template <int NV> struct GxRows {
   gx_rsrc img;
@@ -450,9 +469,9 @@ template <int NV> struct GxRows {
 };
 
 // LDS of a workgroup of NV vector blocks: the ring of stages, then two
-// columns' aux (1 / S and the min-term fragments).
+// columns' aux (1 / S, 4 bytes a lane, and the min-term fragments).
 template <int KIND, int NV> struct GxLds {
-  static constexpr int AUXB = (1 + gx_sums(KIND)) * 1024;
+  static constexpr int INVB = 256, AUXB = INVB + gx_sum_frags(gx_sums(KIND)) * 1024;
   static constexpr int AUX0 = gx_ring(NV) * NV * GX_STAGE, BYTES = AUX0 + 2 * NV * AUXB;
 };
 
@@ -472,7 +491,8 @@ __device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, i
                                            f16v (&acc)[NV]) {
   using U = GxW<KIND>;
   using L = GxLds<KIND, NV>;
-  constexpr int SUMS = gx_sums(KIND), GB = U::GB, AUXN = 1 + SUMS;
+  constexpr int SUMS = gx_sums(KIND), GB = U::GB, AUXN = 1 + gx_sum_frags(SUMS);
+  constexpr bool HALVES = gx_halves(KIND);
   const int lane = threadIdx.x & 63, h = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t ring = __builtin_amdgcn_readfirstlane(lds_offset(lds)), lo16 = 16 * lane;
@@ -497,7 +517,7 @@ __device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, i
     for (int v = 0; v < NV; ++v)
 #pragma unroll
       for (int i = 0; i < AUXN; ++i)
-        if (((v * AUXN + i) & 3) == w) X.aux(v, s, i, dst + v * L::AUXB + 1024 * i);
+        if (((v * AUXN + i) & 3) == w) X.aux(v, s, i, dst + v * L::AUXB + (i ? L::INVB + 1024 * (i - 1) : 0));
   };
   const int row = row0 + (lane & 31), ro = 16 * row;
   U wt;
@@ -527,9 +547,12 @@ __device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, i
       wt.load_head(g0, row, ro, h);
     }
     const auto sc = wt.scales();
-    f16v th[NV], tl[NV];
+    f16v th[NV], tl[NV], t0[NV];
 #pragma unroll
     for (int v = 0; v < NV; ++v) th[v] = tl[v] = zero16();
+    if constexpr (HALVES)
+#pragma unroll
+      for (int v = 0; v < NV; ++v) t0[v] = zero16();
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int g = 4 * c + j;
@@ -573,7 +596,10 @@ __device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, i
 #pragma unroll
             for (int v = 0; v < NV; ++v) tl[v] = mfma3216(lo[v], q, tl[v]);
 #pragma unroll
-            for (int v = 0; v < NV; ++v) th[v] = mfma3216(hi[v], q, th[v]);
+            for (int v = 0; v < NV; ++v) {
+              f16v& t = HALVES && u < 4 ? t0[v] : th[v];
+              t = mfma3216(hi[v], q, t);
+            }
             if constexpr (KIND == Q6_K) {
 #pragma unroll
               for (int v = 0; v < NV; ++v) tl[v] = mfma3216(hi[v], rest, tl[v]);
@@ -602,14 +628,17 @@ __device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, i
 #pragma unroll
       for (int q = 0; q < 4; ++q) inv[q] = *reinterpret_cast<const f4*>(av + 4 * (8 * q + 4 * h));
       f16v tm = zero16();
-      if constexpr (SUMS == 2) tm = mfma3216(*reinterpret_cast<const h8*>(av + 2048 + lo16), m, tm);
-      if constexpr (SUMS != 0) tm = mfma3216(*reinterpret_cast<const h8*>(av + 1024 + lo16), m, tm);
+      if constexpr (SUMS != 0)
+#pragma unroll
+        for (int f = gx_sum_frags(SUMS) - 1; f >= 0; --f)  // the smallest first
+          tm = mfma3216(*reinterpret_cast<const h8*>(av + L::INVB + 1024 * f + lo16), m, tm);
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         float t = th[v][i];
         if constexpr (KIND != Q8_0) {
           t = SUMS != 0 ? __builtin_fmaf(tl[v][i], d, tm[i] * dm) : tl[v][i] * d;
           t = __builtin_fmaf(th[v][i], d, t);
+          if constexpr (HALVES) t = __builtin_fmaf(t0[v][i], d, t);
         }
         acc[v][i] = __builtin_fmaf(t, inv[i >> 2][i & 3], acc[v][i]);
       }

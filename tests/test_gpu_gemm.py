@@ -119,6 +119,81 @@ def test_gemm_infinite_activation(kind):
         assert np.array_equal(Y[35], (-np.inf * W[:, 511]).astype(np.float32), equal_nan=True)
 
 
+def _outliers(X, mode):
+    """Activations with a few dominant ones: one of 1e4 in every vector, seven of
+    1e4, one of 1e4 or four of 1e3 in every column."""
+    X, n = X.copy(), X.shape[1]
+    if mode == "one":
+        X[:, 100] *= np.float32(1e4)
+    elif mode == "seven":
+        X[:, [3, 77, 300, 301, 600, 777, 1000]] *= np.float32(1e4)
+    elif mode == "each":
+        X[:, 100::256] *= np.float32(1e4)
+    elif mode == "four":
+        for j in (5, 60, 130, 200):
+            X[:, j::256] *= np.float32(1e3)
+    return X
+
+
+# The dmin field of the kinds that have one.
+DMIN = {aa.Q4_K: slice(2, 4), aa.Q5_K: slice(2, 4), aa.Q2_K: slice(82, 84)}
+
+
+def _terms(kind, w, in_dim, out_dim):
+    """|d sc q| + |dmin m| of every weight (|w| without a min term): what the two
+    sums of a column add up to before they cancel."""
+    W = oracle.dequant(kind, w, in_dim, out_dim).astype(np.float64)
+    if kind not in DMIN:
+        return np.abs(W)
+    b = w.reshape(-1, aa.BLOCK_BYTES[kind]).copy()
+    b[:, DMIN[kind]] = 0
+    A = oracle.dequant(kind, b.ravel(), in_dim, out_dim).astype(np.float64)
+    return np.abs(A) + np.abs(A - W)
+
+
+@pytest.mark.parametrize("mode", ["one", "seven", "each", "four"])
+@pytest.mark.parametrize("batch", [16, 80])
+@pytest.mark.parametrize("kind", list(aa.KINDS), ids=lambda k: aa.KIND_NAMES[k])
+def test_gemm_outliers(kind, batch, mode):
+    """Dominant activations, within the file's bound over the terms themselves
+    (a sum |w x| of nearly cancelled weights does not bound them).  Rows of 12288:
+    Q4_K and Q6_K take the kernel at 16 vectors too."""
+    out_dim, in_dim = 96, 12288
+    gen = synth.rng(4600 + kind + batch)
+    w = synth.weight_np(kind, out_dim, in_dim, gen)
+    X = _outliers(synth.activations_np(batch * in_dim, gen).reshape(batch, in_dim), mode)
+    Y = _run(kind, w, X, in_dim, out_dim)
+    W = oracle.dequant(kind, w, in_dim, out_dim).astype(np.float64)
+    X64 = X.astype(np.float64)
+    bound = _bound(in_dim) / 4 * (np.abs(X64) @ _terms(kind, w, in_dim, out_dim).T)
+    err = np.abs(Y - X64 @ W.T)
+    assert np.all(err <= bound), f"{mode}: worst err / bound {np.max(err / bound):.3f}"
+
+
+@pytest.mark.parametrize("mode", ["plain", "one", "seven", "each", "four"])
+@pytest.mark.parametrize("batch", [16, 80])
+@pytest.mark.parametrize("kind", [aa.Q5_K, aa.Q3_K, aa.Q2_K, aa.Q8_0], ids=lambda k: aa.KIND_NAMES[k])
+def test_gemm_as_precise_as_the_vector_kernel(kind, batch, mode):
+    """The kinds whose few vectors run on the vector kernel in f32: the error over
+    all outputs against float64 is no larger here on ordinary activations, and
+    stays within a quarter of it beside dominant ones (there the roundings behind
+    the dominant product decide: up to eight of a chain and four of the column's
+    terms, against about ten of the vector kernel's sub-block and quarter)."""
+    out_dim, in_dim = 2048, 1024
+    gen = synth.rng(4700 + kind + batch)
+    w = synth.weight_np(kind, out_dim, in_dim, gen)
+    X = _outliers(synth.activations_np(batch * in_dim, gen).reshape(batch, in_dim), mode)
+    want = X.astype(np.float64) @ oracle.dequant(kind, w, in_dim, out_dim).astype(np.float64).T
+    err = [np.linalg.norm(_run(kind, w, X, in_dim, out_dim) - want)]
+    dev = aa.DeviceOps()
+    dev.set_mm_engine(1)
+    try:
+        err.append(np.linalg.norm(_run(kind, w, X, in_dim, out_dim) - want))
+    finally:
+        dev.set_mm_engine(0)
+    assert err[0] <= (1.0 if mode == "plain" else 1.25) * err[1], f"{err[0] / err[1]:.3f} times the vector kernel's"
+
+
 def test_gemm_replays_in_a_graph():
     """A captured product (columns split, counters re-armed in the kernel)
     replayed with eager products of another shape between the replays."""
