@@ -472,7 +472,10 @@ template <int NV> struct GxRows {
 // columns' aux (1 / S, 4 bytes a lane, and the min-term fragments).
 template <int KIND, int NV> struct GxLds {
   static constexpr int INVB = 256, AUXB = INVB + gx_sum_frags(gx_sums(KIND)) * 1024;
-  static constexpr int AUX0 = gx_ring(NV) * NV * GX_STAGE, BYTES = AUX0 + 2 * NV * AUXB;
+  static constexpr int AUX0 = gx_ring(KIND, NV) * NV * GX_STAGE, BYTES = AUX0 + 2 * NV * AUXB;
+  // Three workgroups (NV = 1) or two per CU in 160 KB, each with 1 KB for what a
+  // kernel has of its own (the ring starts at a multiple of that).
+  static_assert((NV == 1 ? 3 : 2) * (BYTES + 1024) <= 160 * 1024, "workgroups per CU");
 };
 
 // The columns [s0, s1) of 32 rows (rows row0 .. of the 64-row tile whose packed
@@ -496,7 +499,7 @@ __device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, i
   const int lane = threadIdx.x & 63, h = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t ring = __builtin_amdgcn_readfirstlane(lds_offset(lds)), lo16 = 16 * lane;
-  constexpr int R = gx_ring(NV);
+  constexpr int R = gx_ring(KIND, NV);
   const int last = 4 * (s1 - s0) - 1;  // stages
   // Stage g's 8 NV fragments, 2 NV per wave (past the end the last stage
   // again, into a slot nobody reads, so that every stage issues as many).

@@ -12,8 +12,11 @@
 namespace kq {
 
 // 64-element stages (8 KB per vector block) in LDS: as many as leave room for
-// three workgroups per CU (NV = 1) or two (NV = 2).
-__host__ __device__ constexpr int gx_ring(int nv) { return nv == 1 ? 6 : 4; }
+// three workgroups per CU (NV = 1) or two (NV = 2) beside the 1 / S and min
+// sums; Q2_K's three fragments of sums take the room of one stage (with six,
+// two workgroups fit: Q2_K / Q3_K experts at 64 tokens 138 us against 131 with
+// five, Q2_K 14336x4096 x 16 17.7 against 17.4).
+__host__ __device__ constexpr int gx_ring(int kind, int nv) { return nv == 1 ? (kind == Q2_K ? 5 : 6) : 4; }
 
 // Code loads behind stage j: one, two for Q8_0, three in every other one for
 // Q6_K, one in every other one for Q2_K and Q3_K.
@@ -32,7 +35,7 @@ __host__ __device__ constexpr int gx_body_loads(int kind, int j) {
 // that uses it, so those issued in the last column itself (no next one) are not
 // counted there.
 __host__ __device__ constexpr int gx_stage_wait(int kind, int nv, int j, bool last) {
-  const int ahead = gx_ring(nv) - 2;
+  const int ahead = gx_ring(kind, nv) - 2;
   int n = ahead * 2 * nv;
   for (int i = j - ahead; i < j; ++i)
     if (!last || i < 0) n += gx_body_loads(kind, i & 3);

@@ -96,6 +96,6 @@ extern "C" float kq_emul_packed_row(int kind, const uint8_t* g, int lane, const 
 }
 
 // The many-vector core's load stages (kq_gx_stages.h).
-extern "C" int kq_emul_gx_ring(int nv) { return kq::gx_ring(nv); }
+extern "C" int kq_emul_gx_ring(int kind, int nv) { return kq::gx_ring(kind, nv); }
 extern "C" int kq_emul_gx_body_loads(int kind, int j) { return kq::gx_body_loads(kind, j); }
 extern "C" int kq_emul_gx_stage_wait(int kind, int nv, int j, int last) { return kq::gx_stage_wait(kind, nv, j, last != 0); }

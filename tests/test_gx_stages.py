@@ -25,7 +25,7 @@ def emul():
 @pytest.mark.parametrize("nv", [1, 2])
 @pytest.mark.parametrize("kind", aa.KINDS, ids=lambda k: aa.KIND_NAMES[k])
 def test_stage_waits_cover_their_fragments(emul, kind, nv):
-    ring = emul.kq_emul_gx_ring(nv)
+    ring = emul.kq_emul_gx_ring(kind, nv)
     for columns in range(1, 12):
         done, issued = set(range(ring - 1)), []  # the prologue waits for all of its loads
         for g in range(4 * columns):
