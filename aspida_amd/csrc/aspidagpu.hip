@@ -245,18 +245,16 @@ struct HostBuf {
 // to `batch` vectors: the 16-vector kernel, and the 64-vector kernel at each
 // padding (16, 32, 64 vectors) a launch of at most min(batch, 64) vectors
 // takes -- a smaller padding can mean a finer column split and so more
-// partial sums.
-size_t mm_work_bytes(int in_dim, int out_dim, int batch) {
+// partial sums -- and the many-vector kernel's, with any_batch for any number
+// of vectors.
+size_t mm_work_bytes(int in_dim, int out_dim, int batch, bool any_batch) {
   size_t n = kq::mm16_workspace_bytes(in_dim, out_dim);
   for (int bp = 16; bp <= 64; bp *= 2) {
     n = std::max(n, kq::mfma_workspace_bytes(in_dim, out_dim, bp));
     if (bp >= batch) break;
   }
   if (in_dim % 1024 == 0) n = std::max(n, kq::mmw_workspace_bytes(in_dim, out_dim, std::min(batch, 64)));
-  // Room for any batch, so that a stream warmed up with a small one may capture
-  // larger products.
-  n = std::max(n, kq::gemm_workspace_bytes(in_dim, out_dim, kq::GEMM_STEP));
-  return n;
+  return std::max(n, kq::gemm_workspace_bytes(in_dim, out_dim, any_batch ? kq::GEMM_STEP : batch));
 }
 
 // Partial sums and per-tile arrival counters of the packed matvec
@@ -266,10 +264,13 @@ struct MvWorkspace {
   DevBuf<float> part;
   DevBuf<unsigned> count;
   DevBuf<uint8_t> mm;  // activation split and partials of the MFMA product
+  // Room for any batch from the first product on, so that a stream warmed up
+  // with a small one may capture larger products.
+  bool any_batch = true;
   int ensure(int in_dim, int out_dim, int batch = 1) {
     const size_t pf = batch > 1 ? kq::multi_workspace_floats(in_dim, out_dim) : kq::packed_workspace_floats(in_dim, out_dim);
     if (part.ensure(std::max<size_t>(pf, 64), "hipMalloc partials")) return -1;
-    if (batch > 1 && mm.ensure(mm_work_bytes(in_dim, out_dim, batch), "hipMalloc mfma")) return -1;
+    if (batch > 1 && mm.ensure(mm_work_bytes(in_dim, out_dim, batch, any_batch), "hipMalloc mfma")) return -1;
     bool grew = false;
     const size_t nc = kq::packed_counters(out_dim);
     if (count.ensure(batch > 1 ? std::max(nc, kq::GEMM_COUNTERS) : nc, "hipMalloc counters", &grew)) return -1;
@@ -332,7 +333,7 @@ MmRoute mm_route(int kind, int in_dim, int out_dim, int batch) {
   // Q6_K in launches of at most 32 vectors: the 64-vector kernel's Q6_K
   // variant runs out of registers above 32 (14336x4096: 359 us for 64
   // vectors in one launch, 82 us per 32).
-  if (eng == 0 && kq::gemm_takes(kind, in_dim, out_dim, batch)) return {6, kq::GEMM_STEP};
+  if (eng == 0 && kq::gemm_takes(kind, in_dim, out_dim, batch)) return {6, kq::gemm_step(in_dim)};
   if (eng == 4 && kq::mmv_kind(kind)) return {3, 64};
   if (eng == 5 && kq::matvec_nv_takes(kind, in_dim, out_dim)) return {4, 4};
   if (eng == 6 && kq::mmw_takes(kind, in_dim)) return {5, 64};
@@ -419,6 +420,7 @@ struct Ctx {
   Ctx() {
     dx.keep_old = dy.keep_old = dq.keep_old = dh.keep_old = di.keep_old = false;
     ws.part.keep_old = ws.count.keep_old = ws.mm.keep_old = false;
+    ws.any_batch = false;
   }
   int init() {
     if (st) return 0;
@@ -1211,7 +1213,7 @@ extern "C" int aspida_kq_matmul_workspace(int kind, int in_dim, int out_dim, int
                                           long long* needed) {
   if (!valid_kind(kind) || in_dim <= 0 || in_dim % 256 || out_dim <= 0 || batch <= 0 || !allocated || !needed)
     return -EINVAL;
-  *allocated = batch > 1 ? (long long)mm_work_bytes(in_dim, out_dim, batch) : 0;
+  *allocated = batch > 1 ? (long long)mm_work_bytes(in_dim, out_dim, batch, true) : 0;
   *needed = (long long)mm_launch_need(kind, in_dim, out_dim, batch);
   return 0;
 }

@@ -138,6 +138,18 @@ __global__ __launch_bounds__(256, NV == 1 ? 3 : 2) void kq_gemm(GemmArgs a) {
 constexpr int GEMM_WGS = 512;
 constexpr int GEMM_RUNS = 8;
 
+// Offsets within a vector block's image are 31 bits: rows of up to 58254
+// columns.  The image of one call stays below 256 MB where 64 vectors do
+// (512 vectors of up to 455 columns).
+constexpr size_t GEMM_IMAGE = (size_t)256 << 20;
+
+int gemm_step(int in_dim) {
+  const int nsb = in_dim / 256;
+  if (nsb > INT32_MAX / GX_COL) return 0;
+  const size_t pairs = GEMM_IMAGE / ((size_t)2 * nsb * GX_COL);
+  return 64 * (int)std::max<size_t>(1, std::min<size_t>(GEMM_STEP / 64, pairs));
+}
+
 static int gemm_nv(int batch) { return batch > 32 ? 2 : 1; }
 
 static int gemm_ks(int in_dim, int out_dim, int batch) {
@@ -158,6 +170,8 @@ size_t gemm_launch_bytes(int in_dim, int out_dim, int batch) {
 // A split launch has at most GEMM_WGS workgroups of 128 x 64 sums, and never
 // more runs than columns.
 size_t gemm_workspace_bytes(int in_dim, int out_dim, int batch) {
+  batch = std::min(batch, gemm_step(in_dim));
+  if (batch < 1) return 0;
   const size_t cap = (size_t)GEMM_WGS * 128 * 64 * sizeof(float);
   const size_t all = (size_t)(in_dim / 256) * ((out_dim + 127) / 128) * 128 * ((batch + 63) / 64) * 64 * sizeof(float);
   return gemm_image_bytes(in_dim, batch) + std::min(cap, all);
@@ -169,8 +183,7 @@ size_t gemm_workspace_bytes(int in_dim, int out_dim, int batch) {
 // MI355X with every launch of a product counted.
 bool gemm_takes(int kind, int in_dim, int out_dim, int batch) {
   const int nsb = in_dim / 256, tiles = (out_dim + 63) / 64;
-  // Offsets within a vector block's image are 31 bits.
-  if (nsb > INT32_MAX / GX_COL) return false;
+  if (!gemm_step(in_dim)) return false;
   const long units = (long)nsb * tiles;
   // Below 192 tiles (3/4 of a 256-CU device) the one-pass kernel takes 16-row
   // blocks and converts the activations once per 16 rows instead of per 64.
@@ -240,7 +253,7 @@ static hipError_t gemm_launch(const GemmArgs& a, int nv, hipStream_t s) {
 
 hipError_t launch_gemm(int kind, const void* P, int in_dim, int out_dim, int batch, const float* X, float* Y, void* work,
                        unsigned* count, hipStream_t s) {
-  if (batch < 1 || batch > GEMM_STEP) return hipErrorInvalidValue;
+  if (batch < 1 || batch > gemm_step(in_dim)) return hipErrorInvalidValue;
   GemmArgs a{};
   a.P = (const uint8_t*)P;
   a.nsb = in_dim / 256;

@@ -118,11 +118,13 @@ size_t mmw_workspace_bytes(int in_dim, int out_dim, int batch);
 hipError_t launch_matmul_mmw(int kind, const void* P, int in_dim, int out_dim, int batch, const float* X, float* Y,
                              void* work, unsigned* count, hipStream_t s);
 // Products of many vectors over packed weights of every kind (kq_gemm.hip), up
-// to GEMM_STEP vectors per call; `work` holds gemm_launch_bytes, `count`
-// GEMM_COUNTERS unsigned, zero before first use and left zero.  x must be
-// 16-byte aligned.  gemm_takes: where it is the default; gemm_workspace_bytes:
-// what any call of up to `batch` vectors needs.
+// to gemm_step vectors per call (0: rows it does not take); `work` holds
+// gemm_launch_bytes, `count` GEMM_COUNTERS unsigned, zero before first use and
+// left zero.  x must be 16-byte aligned.  gemm_takes: where it is the default;
+// gemm_workspace_bytes: what the calls of any product of up to `batch` vectors
+// need.
 constexpr int GEMM_STEP = 512;
+int gemm_step(int in_dim);
 constexpr size_t GEMM_COUNTERS = 256 * 64;
 bool gemm_takes(int kind, int in_dim, int out_dim, int batch);
 size_t gemm_launch_bytes(int in_dim, int out_dim, int batch);

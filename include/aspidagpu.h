@@ -388,8 +388,8 @@ long long aspida_gguf_read(const aspida_gguf *g, long long i, void *dst, long lo
  * callers leave them at their defaults. */
 
 /* Small-batch workspace check, host only (launches nothing): the bytes of
- * activation split and partial sums the library allocates for a batched
- * product of this kind, shape and batch (*allocated), and the most any single
+ * activation split and partial sums the library allocates on a stream for a
+ * batched product of this kind, shape and batch (*allocated), and the most any single
  * launch of that product uses (*needed).  Returns 0 or -EINVAL. */
 int aspida_kq_matmul_workspace(int kind, int in_dim, int out_dim, int batch, long long *allocated,
                                long long *needed);

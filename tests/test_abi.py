@@ -203,6 +203,22 @@ def test_matmul_of_very_long_rows_keeps_the_vector_kernel(lib):
     assert _matmul_ws(lib, aa.Q5_K, 256 * (longest + 1), 64, 16)[1] == 0
 
 
+@pytest.mark.parametrize("kind", aa.KINDS)
+def test_matmul_workspace_of_long_rows(lib, kind):
+    """The activation image of one launch stays below 256 MB, or that of 64
+    vectors where this is more (36 KB per 32 vectors and column), beside at most
+    16 MB of sums; rows the many-vector kernel does not take reserve nothing for
+    it.  What a product needs is covered either way."""
+    longest = ((1 << 31) - 1) // (36 * 1024)
+    for cols in (455, 456, 1000, 4096, 20000, longest):
+        most = max(256 << 20, 2 * cols * 36 * 1024) + (16 << 20)
+        for batch in (2, 63, 64, 65, 511, 512, 513, 1000):
+            alloc, need = _matmul_ws(lib, kind, 256 * cols, 64, batch)
+            assert need <= alloc <= most, (cols, batch, alloc)
+    over = _matmul_ws(lib, kind, 256 * (longest + 1), 64, 2)[0]
+    assert over <= _matmul_ws(lib, kind, 256 * longest, 64, 2)[0] / 2
+
+
 def test_matmul_workspace_advisor_shapes(lib):
     """The shapes where a 64-row padding undersized the buffer: Q6_K
     8960->1536 at B=48 and Q4_K/Q6_K 3584x3584 at B=48 and 65 -- on the

@@ -119,6 +119,15 @@ def test_gemm_infinite_activation(kind):
         assert np.array_equal(Y[35], (-np.inf * W[:, 511]).astype(np.float32), equal_nan=True)
 
 
+def test_gemm_long_rows():
+    """Rows of 1824 columns, where a launch takes 64 vectors: 66 are two."""
+    batch, out_dim, in_dim = 66, 40, 256 * 1824
+    gen = synth.rng(4550)
+    w = synth.weight_np(aa.Q5_K, out_dim, in_dim, gen)
+    X = synth.activations_np(batch * in_dim, gen).reshape(batch, in_dim)
+    _check(aa.Q5_K, w, X, in_dim, out_dim, "long rows")
+
+
 def _outliers(X, mode):
     """Activations with a few dominant ones: one of 1e4 in every vector, seven of
     1e4, one of 1e4 or four of 1e3 in every column."""
