@@ -207,14 +207,23 @@ bool gemm_takes(int kind, int in_dim, int out_dim, int batch) {
     }
     // Q6_K 33..64: 14336x4096 35.2 / 88.6, 4096^2 21.1 / 27.6, 1024x2048 16.2 /
     // 25.4; the wave-per-column kernel is ahead on few tiles of long rows up to
-    // 48 (1024x14336 at 33: 32.9 / 29.9, at 64: 33.2 / 40.4).
-    if (batch > 32) return batch > 48 || units > 1024 || nsb < 32;
+    // 48 (1024x14336 at 33: 32.9 / 29.9, at 64: 33.2 / 40.4), and so are two
+    // launches of the one-pass kernel on few tiles of two columns, which a split
+    // into runs does not shorten (4096x512 at 33: 11.7 / 9.5, at 48 11.8 / 10.1,
+    // at 52 11.8 / 12.1, but 16384x512 at 33 13.4 / 25.7; one column: 8.6 / 8.8,
+    // three: 12.0 / 21.2).
+    if (batch > 32) return batch > 48 || units > 1024 || (nsb < 32 && (nsb != 2 || units >= 256));
     // 17..32: 4096^2 15.0 / 19.9, 1024x4096 14.1 / 18.7, but 2048^2 12.1 / 11.1.
     if (batch > 16) return nsb >= 16;
     const bool split16 = narrow && tiles >= 128 && nsb >= 16;  // 8192x4096 18.0 / 19.8 at 6
-    // 9..16: 14336x4096 23.8 / 27.2 and 1024x14336 21.8 / 33.2 at 12, 4096^2
-    // 14.6 / 16.7 at 16 but 14.6 / 13.3 at 12.
-    if (batch > 8) return units >= 3584 || nsb >= 48 || split16 || (batch > 12 && nsb >= 16);
+    // 9..16: 14336x4096 23.8 / 27.2 and 1024x14336 21.8 / 33.2 at 12.  From 13 on
+    // rows of more than 16 columns (4096x5120 17.0 / 22.8 at 13, 4096x6144 17.0 /
+    // 17.1 at 14, 1024x8192 18.2 / 20.5 at 13); at 16 columns, one for each of the
+    // one-pass kernel's waves, only where its 16-row blocks are more than the CUs
+    // (6144x4096 17.2 / 24.7 at 15) or for 16 vectors (4096^2 14.3 / 16.0 at 16
+    // but 14.5 / 12.2 at 13, 14.4 / 13.3 at 15).
+    if (batch > 8)
+      return units >= 3584 || nsb >= 48 || split16 || (batch > 12 && nsb >= 16 && (nsb > 16 || tiles > 64 || batch > 15));
     // 5..8: 28672x4096 36.5 / 41.3, 8192^2 25.8 / 34.0, 4096x14336 28.0 / 29.4,
     // but 14336x4096 23.6 / 22.6 and 4096x8192 20.3 / 18.9.
     if (batch > 4) return units >= 7168 || nsb >= 48 || split16;
@@ -222,9 +231,11 @@ bool gemm_takes(int kind, int in_dim, int out_dim, int batch) {
   }
   // The others' path is the vector kernel, 8 vectors a launch: 4096^2 Q5_K
   // 14.0 / 43.5 at 16, Q8_0 14.2 / 20.3 at 8, Q2_K 13.5 / 17.6 at 8; at 5
-  // vectors 14.0 / 16.4 (Q5_K), 13.8 / 13.3 (Q2_K).  Products too small to fill
-  // a wave's columns stay there up to three launches of it, where each row is
-  // the batch-1 vector kernel's bit for bit.
+  // vectors 14.0 / 16.4 (Q5_K), 13.8 / 13.3 (Q2_K).  Up to three launches of it
+  // below 16 units stay there for their bits, not for the time: each row is the
+  // batch-1 vector kernel's, on products that do not fill one workgroup a CU
+  // either way (Q5_K 200x512 8.8 / 19.3 at 8, 9.1 / 57.6 at 24; 64x256 6.6 / 11.2
+  // at 5).
   if (units < 16 && batch <= 24) return false;
   if (batch >= 8) return true;
   // 1024x14336 at 6: Q5_K 20.9 / 22.2, Q2_K 19.9 / 18.3, Q8_0 21.3 / 20.2.

@@ -412,12 +412,13 @@ def gemm_takes(aa, kind, inp, out, B):
             return nsb >= 16 or units >= 3584
         return B > 4 and narrow and (units >= (2048 if B > 8 else 3584) or nsb >= 48)
     if B > 32:
-        return B > 48 or units > 1024 or nsb < 32
+        return B > 48 or units > 1024 or (nsb < 32 and (nsb != 2 or units >= 256))
     if B > 16:
         return nsb >= 16
     split16 = narrow and tiles >= 128 and nsb >= 16
     if B > 8:
-        return units >= 3584 or nsb >= 48 or split16 or (B > 12 and nsb >= 16)
+        return units >= 3584 or nsb >= 48 or split16 or \
+            (B > 12 and nsb >= 16 and (nsb > 16 or tiles > 64 or B > 15))
     if B > 4:
         return units >= 7168 or nsb >= 48 or split16
     return B > 2 and units >= 16384

@@ -203,6 +203,44 @@ def test_matmul_of_very_long_rows_keeps_the_vector_kernel(lib):
     assert _matmul_ws(lib, aa.Q5_K, 256 * (longest + 1), 64, 16)[1] == 0
 
 
+def _on_many_vector_kernel(lib, kind, in_dim, out_dim, batch):
+    """Whether a product of 2 to 512 vectors runs on the many-vector kernel, by
+    what its launch needs: an activation image of 36 KB per 32 vectors and column,
+    and the sums of ks runs of columns over groups of 128 rows and 32 or 64
+    vectors (no other kernel's need is of that size)."""
+    cols, per = in_dim // 256, 32 if batch <= 32 else 64
+    tiles = -(-out_dim // 128) * -(-batch // per)
+    ks = max(1, min(cols, 512 // tiles, max(8, in_dim // 1024)))
+    image = -(-batch // 32) * cols * 36 * 1024
+    return _matmul_ws(lib, kind, in_dim, out_dim, batch)[1] == image + (ks * tiles * 128 * per * 4 if ks > 1 else 0)
+
+
+def test_many_vector_kernel_not_where_it_is_slower(lib):
+    """Q6_K products on which the one-pass kernel measured ahead of the
+    many-vector kernel stay on it: 13 to 15 vectors of 16 columns, 33 to 48 of two
+    columns on few tiles; their neighbours do not."""
+    takes = lambda *a: _on_many_vector_kernel(lib, aa.Q6_K, *a)
+    for out_dim in (1024, 3072, 4096):
+        assert [takes(4096, out_dim, b) for b in (12, 13, 14, 15, 16, 17)] == [False] * 4 + [True] * 2
+        assert takes(5120, out_dim, 13) and takes(8192, out_dim, 13)
+    assert takes(4096, 4160, 13) and takes(4096, 6144, 13)
+    for out_dim in (64, 960, 4096):
+        assert [takes(512, out_dim, b) for b in (33, 40, 48, 49, 64, 65)] == [False] * 3 + [True] * 3
+        assert takes(256, out_dim, 33) and takes(768, out_dim, 33)
+    assert takes(512, 16384, 33)
+
+
+def test_bench_names_the_kernel_the_library_picks(lib):
+    """bench.py's statement of the rule (gemm_takes) is the library's."""
+    import bench
+    for kind in (aa.Q4_K, aa.Q6_K):
+        for in_dim in (256, 512, 768, 2048, 3072, 4096, 4352, 6144, 8192, 12288, 14336):
+            for out_dim in (64, 320, 1024, 4096, 4160, 8192, 8256, 12288, 14336, 28672, 65536):
+                for b in (2, 3, 4, 5, 8, 9, 12, 13, 15, 16, 17, 32, 33, 48, 49, 64, 65, 300):
+                    want = bench.gemm_takes(aa, kind, in_dim, out_dim, b)
+                    assert _on_many_vector_kernel(lib, kind, in_dim, out_dim, b) == want, (kind, in_dim, out_dim, b)
+
+
 @pytest.mark.parametrize("kind", aa.KINDS)
 def test_matmul_workspace_of_long_rows(lib, kind):
     """The activation image of one launch stays below 256 MB, or that of 64
