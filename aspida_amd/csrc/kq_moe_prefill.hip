@@ -305,13 +305,19 @@ bool moe_prefill_takes(int T, int gu_kind, int down_kind, int dim, int I, int to
   if (!gx_may_take(T, dim, I) || gu_kind < 0 || gu_kind > Q8_0 || down_kind < 0 || down_kind > Q8_0 || top_k < 1 || top_k > MOE_MAX_TOPK || n_exp < 1 || n_exp > MOE_MAX_EXP ||
       t * (top_k + 1) * (I / 256) * GX_REC >= (size_t)1 << 32 || t * (dim / 256) * GX_REC >= (size_t)1 << 32)
     return false;
-  // Q4_K / Q6_K, 2048x768, 128 experts, top 8: 175 / 296 at 95 tokens.
-  if (T >= 96) return true;
   const long jobs = (long)T * top_k;
   // Q4_K / Q6_K: at 48 tokens 2048x768 with 128 experts, top 8 161 / 172; with
   // 60, top 4 91 / 99; with 16, top 2 63 / 69 (at 32: 150 / 126, 90 / 77, 63 /
   // 55).  Many jobs per expert pay earlier: 16 experts, top 8 61 / 67 at 16.
-  if (moe_mfma_kind(gu_kind) && moe_mfma_kind(down_kind)) return T >= 48 || (T >= 16 && jobs >= 6L * n_exp);
+  // Fewer than about two per expert, the shared one's counted too, do not pay at
+  // any T: a group then holds what two chunks do.  Experts alone, Q4_K / Q4_K
+  // 2048x768: 128 experts, top 2 75 / 63 at 48 tokens, 87 / 83 at 72, 97 / 106 at
+  // 95; top 3 88 / 79 at 48, 100 / 106 at 72; top 4 97 / 90 at 48, 105 / 111 at
+  // 64; 256 experts, top 2 129 / 115 at 96, 153 / 144 at 128, 183 / 202 at 200.
+  // Below 56 tokens three: 1024x512, 128 experts, top 5, Q4_K / Q6_K 51 / 49 at
+  // 48, 51 / 53 at 56, and 64 experts, top 3, 1024x768 45 / 48 at 48.
+  if (moe_mfma_kind(gu_kind) && moe_mfma_kind(down_kind))
+    return (T >= 48 && 4 * (jobs + T) >= (T < 56 ? 12L : 9L) * n_exp) || (T >= 16 && jobs >= 6L * n_exp);
   // Others: 128 experts, top 8 at 16 tokens Q5_K/Q6_K 122 / 139, Q2_K/Q3_K 103 /
   // 110 (at 8: 96 / 90, 83 / 74); 16 experts, top 8 at 4 tokens Q5_K/Q6_K 54 / 66.
   return T >= 16 || jobs >= 2L * n_exp;

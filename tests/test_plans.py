@@ -7,6 +7,8 @@ comment names the measurement it rests on.  The tuple is (matrix cores, waves
 per workgroup, workgroups per 64-row tile, columns per wave, columns one after
 another, 16-row workgroups).
 """
+import ctypes
+
 import pytest
 
 import aspida_amd as aa
@@ -85,3 +87,39 @@ def test_overrides_are_per_thread(dev):
     assert seen["rows"][5] is False and seen["rows"][0]   # 64-row workgroups in that thread
     assert seen["engine"] is False                         # vector engine in that thread
     assert dev.matvec_plan(aa.Q4_K, 4096, 4096) == (True, 16, 1, 1, False, True)  # untouched here
+
+
+def _many_jobs(T, gu, down, dim, inter, top_k, n_exp):
+    """moe_prefill_takes (kq_moe.h): whether the experts run as the grouped
+    many-job products."""
+    takes = aa.load()._ZN2kq17moe_prefill_takesEiiiiiii
+    takes.restype = ctypes.c_bool
+    return takes(T, gu, down, dim, inter, top_k, n_exp)
+
+
+# dim, inter, experts, top k: tokens (kinds on the chunked matrix-core path) from
+# which the many-job products measured ahead, and a count below that at which the
+# chunked path is.
+MOE_LINES = [
+    ((2048, 768, 128, 2), 96, 80),     # Q4_K / Q4_K 96 us vs 103; 91 vs 88
+    ((2048, 768, 128, 3), 72, 56),     # 100 vs 106; 91 vs 84
+    ((2048, 768, 128, 4), 64, 48),     # 105 vs 111; 97 vs 90
+    ((2048, 768, 128, 8), 48, 40),     # 128 vs 150
+    ((1536, 512, 128, 2), 96, 80),     # 59 vs 60; 55 vs 51
+    ((2048, 768, 256, 2), 200, 128),   # 183 vs 202; 153 vs 144
+    ((2048, 768, 256, 8), 72, 56),     # 202 vs 225; 189 vs 182
+    ((2048, 768, 60, 4), 48, 40),      # 68 vs 82
+    ((1024, 768, 64, 3), 48, 40),      # 41 vs 47
+    ((1024, 512, 128, 5), 56, 48),     # 49 vs 50; 49 vs 46
+    ((2048, 768, 64, 2), 56, 48),      # 62 vs 64; 61 vs 59
+]
+
+
+@pytest.mark.parametrize("shape,first,below", MOE_LINES)
+@pytest.mark.parametrize("kinds", [(aa.Q4_K, aa.Q6_K), (aa.Q4_K, aa.Q4_K), (aa.Q6_K, aa.Q6_K)])
+def test_moe_few_jobs_per_expert_stay_on_the_chunked_path(kinds, shape, first, below):
+    dim, inter, n_exp, top_k = shape
+    for T in (1, 2, below - 8, below):
+        assert not _many_jobs(T, *kinds, dim, inter, top_k, n_exp), T
+    for T in (first, first + 8, 512, 1024, 4096):
+        assert _many_jobs(T, *kinds, dim, inter, top_k, n_exp), T
