@@ -330,10 +330,10 @@ MmRoute mm_route(int kind, int in_dim, int out_dim, int batch) {
                     (eng == 3 || (eng == 0 && batch > MULTI_MAX_BATCH_MFMA_KINDS &&
                                   (batch <= 16 || (units >= MM16_MIN_UNITS && kind != kq::Q4_K))));
   const bool mm64 = !mm16 && kq::mfma_kind(kind) && (eng == 2 || (eng == 0 && batch > MULTI_MAX_BATCH_MFMA_KINDS));
-  // Q6_K in launches of at most 32 vectors: the 64-vector kernel's Q6_K
-  // variant runs out of registers above 32 (14336x4096: 359 us for 64
-  // vectors in one launch, 82 us per 32).
-  if (eng == 0 && kq::gemm_takes(kind, in_dim, out_dim, batch)) return {6, kq::gemm_step(in_dim)};
+  // Under aspida_kq_set_mv_engine(1) the other kinds' products keep the batch-1
+  // vector kernel's bits at any batch, as the MoE layer keeps its kernels.
+  if (eng == 0 && kq::matvec_engine() == 0 && kq::gemm_takes(kind, in_dim, out_dim, batch))
+    return {6, kq::gemm_step(in_dim)};
   if (eng == 4 && kq::mmv_kind(kind)) return {3, 64};
   if (eng == 5 && kq::matvec_nv_takes(kind, in_dim, out_dim)) return {4, 4};
   if (eng == 6 && kq::mmw_takes(kind, in_dim)) return {5, 64};
@@ -356,6 +356,9 @@ MmRoute mm_route(int kind, int in_dim, int out_dim, int batch) {
     if (batch <= 16 || kind == kq::Q6_K) return {3, kq::mmv_step(kind, in_dim, out_dim)};
   }
   if (mm16) return {1, 16};
+  // Q6_K in launches of at most 32 vectors: the 64-vector kernel's Q6_K
+  // variant runs out of registers above 32 (14336x4096: 359 us for 64
+  // vectors in one launch, 82 us per 32).
   if (mm64) return {2, kind == kq::Q6_K ? 32 : 64};
   return {0, MULTI_MAX_BATCH};
 }

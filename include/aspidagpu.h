@@ -155,7 +155,9 @@ int aspida_kq_matvec2_packed_dev(int kind_a, const void *packed_a, int out_a, fl
  * scales), up to 512 vectors per weight pass, except few vectors of Q5_K,
  * Q3_K, Q2_K and Q8_0 (up to 4 to 7 by shape, 24 on the smallest matrices),
  * which run on the vector kernel, each row bit-identical to
- * aspida_kq_matvec_packed_dev on it under aspida_kq_set_mv_engine(1).
+ * aspida_kq_matvec_packed_dev on it (aspida_kq_set_mv_engine(1)).  A row's
+ * bits otherwise depend on how many vectors the product has; while that
+ * override is set, these four kinds run there for any batch.
  * x must be 16-byte aligned; workspace as for aspida_kq_matvec_packed_dev
  * (sized by in_dim and out_dim, the many-vector part for any batch).
  * The same math as the reference's batched kernels (gpu/gpu_matvec.cu:234-382)
@@ -401,9 +403,9 @@ int aspida_kq_matmul_workspace(int kind, int in_dim, int out_dim, int batch, lon
 int aspida_kq_set_packed_plan(int waves_per_group, int groups_per_tile);
 
 /* Engine of the batch-1 packed matvec (aspida_kq_matvec_packed_dev and the
- * calls built on it): 0 = matrix cores (MFMA) for Q4_K and Q6_K, the vector
- * kernel for the other kinds (the default); 1 = the vector kernel for every
- * kind.
+ * calls built on it): 0 = matrix cores (MFMA) for the five K-quants, the vector
+ * kernel for Q8_0 (the default); 1 = the vector kernel for every kind, and no
+ * many-job MoE or many-vector product.
  * Per calling thread; for comparison and tests.  No reference counterpart.
  * Returns 0, or -EINVAL for another value. */
 int aspida_kq_set_mv_engine(int engine);

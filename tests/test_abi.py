@@ -230,6 +230,17 @@ def test_many_vector_kernel_not_where_it_is_slower(lib):
     assert takes(512, 16384, 33)
 
 
+@pytest.mark.parametrize("kind", [aa.Q5_K, aa.Q3_K, aa.Q2_K, aa.Q8_0])
+def test_vector_engine_takes_products_off_the_many_vector_kernel(lib, kind):
+    assert _on_many_vector_kernel(lib, kind, 4096, 4096, 16)
+    assert lib.aspida_kq_set_mv_engine(1) == 0
+    try:
+        for batch in (2, 16, 64, 300):
+            assert _matmul_ws(lib, kind, 4096, 4096, batch)[1] == 0
+    finally:
+        assert lib.aspida_kq_set_mv_engine(0) == 0
+
+
 def test_bench_names_the_kernel_the_library_picks(lib):
     """bench.py's statement of the rule (gemm_takes) is the library's."""
     import bench

@@ -119,6 +119,25 @@ def test_gemm_infinite_activation(kind):
         assert np.array_equal(Y[35], (-np.inf * W[:, 511]).astype(np.float32), equal_nan=True)
 
 
+@pytest.mark.parametrize("kind", [aa.Q5_K, aa.Q3_K, aa.Q2_K, aa.Q8_0], ids=lambda k: aa.KIND_NAMES[k])
+def test_vector_engine_keeps_the_rows_bits_at_any_batch(kind):
+    """Under set_mv_engine(1) every row of a product is the one-vector call's bit
+    for bit, also where the library's own pick is the many-vector kernel."""
+    out_dim, in_dim = 520, 1024
+    gen = synth.rng(4560 + kind)
+    w = synth.weight_np(kind, out_dim, in_dim, gen)
+    X = synth.activations_np(70 * in_dim, gen).reshape(70, in_dim)
+    dev = aa.DeviceOps()
+    dev.set_mv_engine(1)
+    try:
+        rows = np.stack([_run(kind, w, X[b:b + 1], in_dim, out_dim)[0] for b in range(70)])
+        for batch in (2, 8, 19, 70):
+            Y = _run(kind, w, X[:batch], in_dim, out_dim)
+            assert np.array_equal(Y.view(np.uint32), rows[:batch].view(np.uint32)), batch
+    finally:
+        dev.set_mv_engine(0)
+
+
 def test_gemm_long_rows():
     """Rows of 1824 columns, where a launch takes 64 vectors: 66 are two."""
     batch, out_dim, in_dim = 66, 40, 256 * 1824
