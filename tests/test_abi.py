@@ -204,15 +204,35 @@ def test_matmul_of_very_long_rows_keeps_the_vector_kernel(lib):
 
 
 def _on_many_vector_kernel(lib, kind, in_dim, out_dim, batch):
-    """Whether a product of 2 to 512 vectors runs on the many-vector kernel, by
-    what its launch needs: an activation image of 36 KB per 32 vectors and column,
+    """Whether a product runs on the many-vector kernel, by what its launches of up
+    to 512 vectors need: an activation image of 36 KB per 32 vectors and column,
     and the sums of ks runs of columns over groups of 128 rows and 32 or 64
     vectors (no other kernel's need is of that size)."""
-    cols, per = in_dim // 256, 32 if batch <= 32 else 64
-    tiles = -(-out_dim // 128) * -(-batch // per)
-    ks = max(1, min(cols, 512 // tiles, max(8, in_dim // 1024)))
-    image = -(-batch // 32) * cols * 36 * 1024
-    return _matmul_ws(lib, kind, in_dim, out_dim, batch)[1] == image + (ks * tiles * 128 * per * 4 if ks > 1 else 0)
+    def launch(n):
+        cols, per = in_dim // 256, 32 if n <= 32 else 64
+        tiles = -(-out_dim // 128) * -(-n // per)
+        ks = max(1, min(cols, 512 // tiles, max(8, in_dim // 1024)))
+        return -(-n // 32) * cols * 36 * 1024 + (ks * tiles * 128 * per * 4 if ks > 1 else 0)
+
+    need = max([launch(min(batch, 512))] + ([launch(batch % 512)] if batch > 512 and batch % 512 else []))
+    return _matmul_ws(lib, kind, in_dim, out_dim, batch)[1] == need
+
+
+def test_many_vector_cases_run_on_the_kernel(lib):
+    """The GPU tests of the many-vector kernel call the library's own pick: it is
+    that kernel for every kind, but for Q4_K and Q6_K at the few-vector cases named
+    there, and at the shapes of the other tests of that file."""
+    from test_gpu_gemm import CASES
+    few = [(25, 130, 256), (32, 33, 2304), (33, 200, 512)]
+    for kind in aa.KINDS:
+        for batch, out_dim, in_dim in CASES:
+            elsewhere = kind in (aa.Q4_K, aa.Q6_K) and (batch, out_dim, in_dim) in few
+            assert _on_many_vector_kernel(lib, kind, in_dim, out_dim, batch) != elsewhere, (kind, batch, out_dim, in_dim)
+        for batch, out_dim, in_dim in [(72, 160, 1024), (66, 96, 512), (16, 96, 12288), (80, 96, 12288)]:
+            assert _on_many_vector_kernel(lib, kind, in_dim, out_dim, batch), (kind, batch, out_dim, in_dim)
+    for kind in (aa.Q5_K, aa.Q3_K, aa.Q2_K, aa.Q8_0):
+        for batch, out_dim, in_dim in [(40, 96, 768), (16, 2048, 1024), (80, 2048, 1024), (40, 384, 2048)]:
+            assert _on_many_vector_kernel(lib, kind, in_dim, out_dim, batch), (kind, batch, out_dim, in_dim)
 
 
 def test_many_vector_kernel_not_where_it_is_slower(lib):

@@ -173,7 +173,9 @@ def test_multi_vector_rows_bit_identical_to_matvec(kind, case):
 
 @pytest.mark.parametrize("kind", [aa.Q5_K, aa.Q8_0])
 def test_multi_vector_chunks_beyond_eight(kind):
-    """Kinds without MFMA run batches above 8 as launches of 8."""
+    """Products of the kinds without a small-batch MFMA kernel that stay on the
+    vector kernel (8 (tile, column) units here, below 16) run batches above 8 as
+    launches of 8."""
     batch, out_dim, in_dim = 19, 200, 512
     gen = synth.rng(811 + kind)
     w = synth.weight_np(kind, out_dim, in_dim, gen)

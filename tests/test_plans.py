@@ -123,3 +123,11 @@ def test_moe_few_jobs_per_expert_stay_on_the_chunked_path(kinds, shape, first, b
         assert not _many_jobs(T, *kinds, dim, inter, top_k, n_exp), T
     for T in (first, first + 8, 512, 1024, 4096):
         assert _many_jobs(T, *kinds, dim, inter, top_k, n_exp), T
+
+
+def test_moe_many_job_cases_take_their_path():
+    """The GPU tests of the many-job products call the library's own pick."""
+    from test_gpu_moe_many import CASES
+    for dim, inter, n_exp, top_k, gk, dk, _, T, _ in CASES + [(1024, 512, 6, 3, aa.Q5_K, aa.Q6_K, True, 20, 0),
+                                                              (1024, 512, 16, 6, aa.Q4_K, aa.Q6_K, True, 16, 0)]:
+        assert _many_jobs(T, gk, dk, dim, inter, top_k, n_exp), (dim, inter, n_exp, top_k, T)
