@@ -85,20 +85,15 @@ __device__ __forceinline__ h8 gx_ints(uint32_t a, uint32_t b, uint32_t c, uint32
 __device__ __forceinline__ uint32_t byte_of(uint32_t lo, uint32_t hi, int i) { return bfe(i < 4 ? lo : hi, 8 * (i & 3), 8); }
 
 // A lane's share of one super-block column of a 32-row block: its `head`
-// (scales; loaded a column ahead) and `body` (codes).  P = uint4 holds the
-// pieces of both steps b = 0, 1 of a sub-block pair, uint2 those of one (8
-// bytes of each chunk).  load_head / load_body(j) read the column at g for
-// tile row `row`, pieces at chunk offset ro = 16 row (+ 8 b); body(j) is what
-// stage j (u = 2j, 2j + 1) was the last to use.  frag(u, b) is the B operand
-// of step 2u + b.
-template <int KIND, class P = uint4> struct GxW;
+// (scales; loaded a column ahead) and `body` (codes).  A 16-byte piece of its
+// row holds both steps b = 0, 1 of a sub-block pair.  load_head / load_body(j)
+// read the column at g for tile row `row`, pieces at chunk offset ro = 16 row;
+// body(j) is what stage j (u = 2j, 2j + 1) was the last to use.  frag(u, b) is
+// the B operand of step 2u + b.
+template <int KIND> struct GxW;
 
 __device__ __forceinline__ uint32_t first(const uint4& v, int b) { return b ? v.z : v.x; }
 __device__ __forceinline__ uint32_t second(const uint4& v, int b) { return b ? v.w : v.y; }
-__device__ __forceinline__ uint32_t first(const uint2& v, int) { return v.x; }
-__device__ __forceinline__ uint32_t second(const uint2& v, int) { return v.y; }
-__device__ __forceinline__ void gx_ld(uint4& v, const uint8_t* p) { v = ld16(p); }
-__device__ __forceinline__ void gx_ld(uint2& v, const uint8_t* p) { v = ld8(p); }
 
 // Q4_K and Q5_K scales and mins as bytes: s[0..3], s[4..7], m[0..3], m[4..7].
 struct GxScaleMin {
@@ -113,17 +108,17 @@ struct GxScaleMin {
   }
 };
 
-template <class P> struct GxW<Q4_K, P> {
+template <> struct GxW<Q4_K> {
   static constexpr int GB = 64 * 144;
   uint4 hd, hn;
-  P q[4];
+  uint4 q[4];
   __device__ __forceinline__ void load_head(const uint8_t* g, int row, int, int) { hn = ld16(g + 16 * row); }
   __device__ __forceinline__ void next_head() { hd = hn; }
   __device__ __forceinline__ void load_body(const uint8_t* g, int ro, int h, int j) {
-    gx_ld(q[j], g + (1 + 2 * j + h) * 1024 + ro);
+    q[j] = ld16(g + (1 + 2 * j + h) * 1024 + ro);
   }
   __device__ __forceinline__ h8 frag(const GxScaleMin& sm, int u, int b, int) const {
-    const P& c = q[u >> 1];
+    const uint4& c = q[u >> 1];
     const uint32_t x = first(c, b), y = second(c, b), m = u & 1 ? 0x00F000F0u : 0x000F000Fu;
     return as_h8(x & m, (x >> 8) & m, y & m, (y >> 8) & m) * sm.scale(u, u & 1 ? 64.f : 1024.f);
   }
@@ -132,23 +127,23 @@ template <class P> struct GxW<Q4_K, P> {
   __device__ __forceinline__ float dmin() const { return f16_ada(hd.x >> 16); }
 };
 
-template <class P> struct GxW<Q5_K, P> {
+template <> struct GxW<Q5_K> {
   static constexpr int GB = 64 * 176;
   uint4 hd, hn;
-  P qh, qhn, q[4];
+  uint4 qh, qhn, q[4];
   __device__ __forceinline__ void load_head(const uint8_t* g, int row, int ro, int h) {
     hn = ld16(g + 16 * row);
-    gx_ld(qhn, g + (1 + h) * 1024 + ro);
+    qhn = ld16(g + (1 + h) * 1024 + ro);
   }
   __device__ __forceinline__ void next_head() {
     hd = hn;
     qh = qhn;
   }
   __device__ __forceinline__ void load_body(const uint8_t* g, int ro, int h, int j) {
-    gx_ld(q[j], g + (3 + 2 * j + h) * 1024 + ro);
+    q[j] = ld16(g + (3 + 2 * j + h) * 1024 + ro);
   }
   __device__ __forceinline__ h8 frag(const GxScaleMin& sm, int u, int b, int) const {
-    const P& c = q[u >> 1];
+    const uint4& c = q[u >> 1];
     const uint32_t x = first(c, b) >> (4 * (u & 1)), y = (second(c, b)) >> (4 * (u & 1));
     const uint32_t hx = first(qh, b), hy = second(qh, b);
     const uint32_t tx = u < 4 ? hx << (4 - u) : hx >> (u - 4), ty = u < 4 ? hy << (4 - u) : hy >> (u - 4);
@@ -163,7 +158,7 @@ template <class P> struct GxW<Q5_K, P> {
 
 // Q2_K: 16 (scale, min) nibble pairs in chunk 0, scale 2u + h of sub-block
 // (u, h); codes 2 bits at shift 2 (u % 4) of chunk 1 + 2 (u / 4) + h.
-template <class P> struct GxW<Q2_K, P> {
+template <> struct GxW<Q2_K> {
   static constexpr int GB = 64 * 84;
   struct S {
     uint4 s;
@@ -178,7 +173,7 @@ template <class P> struct GxW<Q2_K, P> {
     }
   };
   uint4 sc, scn;
-  P q[2];
+  uint4 q[2];
   uint32_t dd, ddn;
   __device__ __forceinline__ void load_head(const uint8_t* g, int row, int, int) {
     scn = ld16(g + 16 * row);
@@ -189,10 +184,10 @@ template <class P> struct GxW<Q2_K, P> {
     dd = ddn;
   }
   __device__ __forceinline__ void load_body(const uint8_t* g, int ro, int h, int j) {
-    if (j & 1) gx_ld(q[j >> 1], g + (1 + 2 * (j >> 1) + h) * 1024 + ro);
+    if (j & 1) q[j >> 1] = ld16(g + (1 + 2 * (j >> 1) + h) * 1024 + ro);
   }
   __device__ __forceinline__ h8 frag(const S& s, int u, int b, int h) const {
-    const P& c = q[u >> 2];
+    const uint4& c = q[u >> 2];
     const uint32_t x = first(c, b), y = second(c, b), m = 0x00030003u << (2 * (u & 3));
     return as_h8(x & m, (x >> 8) & m, y & m, (y >> 8) & m) * s.scale(u, h);
   }
@@ -203,7 +198,7 @@ template <class P> struct GxW<Q2_K, P> {
 
 // Q3_K: 6-bit scales of 16 elements, code = low2 + 4 hbit - 4; hmask bit u of
 // chunk h, codes at shift 2 (u % 4) of chunk 2 + 2 (u / 4) + h.
-template <class P> struct GxW<Q3_K, P> {
+template <> struct GxW<Q3_K> {
   static constexpr int GB = 64 * 110;
   struct S {
     uint32_t s[4];
@@ -211,10 +206,10 @@ template <class P> struct GxW<Q3_K, P> {
       return splat8((float)((int)((s[u >> 1] >> (16 * (u & 1) + 8 * h)) & 0xFFu) - 32) * 1024.f);
     }
   };
-  P hm, hmn, q[2];
+  uint4 hm, hmn, q[2];
   uint32_t a0, a1, a2, dd, b0, b1, b2, ddn;
   __device__ __forceinline__ void load_head(const uint8_t* g, int row, int ro, int h) {
-    gx_ld(hmn, g + h * 1024 + ro);
+    hmn = ld16(g + h * 1024 + ro);
     const uint8_t* sp = g + 6 * 1024 + 12 * row;
     b0 = ld4(sp);
     b1 = ld4(sp + 4);
@@ -229,10 +224,10 @@ template <class P> struct GxW<Q3_K, P> {
     dd = ddn;
   }
   __device__ __forceinline__ void load_body(const uint8_t* g, int ro, int h, int j) {
-    if (j & 1) gx_ld(q[j >> 1], g + (2 + 2 * (j >> 1) + h) * 1024 + ro);
+    if (j & 1) q[j >> 1] = ld16(g + (2 + 2 * (j >> 1) + h) * 1024 + ro);
   }
   __device__ __forceinline__ h8 frag(const S& s, int u, int b, int h) const {
-    const P& c = q[u >> 2];
+    const uint4& c = q[u >> 2];
     const uint32_t x = first(c, b) >> (2 * (u & 3)), y = (second(c, b)) >> (2 * (u & 3));
     const uint32_t hx = first(hm, b), hy = second(hm, b);
     const uint32_t tx = u < 2 ? hx << (2 - u) : hx >> (u - 2), ty = u < 2 ? hy << (2 - u) : hy >> (u - 2);
@@ -253,7 +248,7 @@ template <class P> struct GxW<Q3_K, P> {
 // 4 hh + 2 (k % 2) + h, the two high bits at shift 2 k of chunk 8 + 2 hh + h,
 // and the int8 scale 2 u + h.  frag gives the product's f16 rounding, rest
 // what it leaves.
-template <class P> struct GxW<Q6_K, P> {
+template <> struct GxW<Q6_K> {
   static constexpr int GB = 64 * 210;
   struct S {
     uint4 s;
@@ -263,7 +258,7 @@ template <class P> struct GxW<Q6_K, P> {
     }
   };
   uint4 sc, scn;
-  P qa[2], qb[2], qh[2];
+  uint4 qa[2], qb[2], qh[2];
   uint32_t dd, ddn;
   __device__ __forceinline__ void load_head(const uint8_t* g, int row, int, int) {
     scn = ld16(g + 12 * 1024 + 16 * row);
@@ -276,9 +271,9 @@ template <class P> struct GxW<Q6_K, P> {
   __device__ __forceinline__ void load_body(const uint8_t* g, int ro, int h, int j) {
     if (j & 1) {
       const int hh = j >> 1;
-      gx_ld(qa[hh], g + (4 * hh + h) * 1024 + ro);
-      gx_ld(qb[hh], g + (4 * hh + 2 + h) * 1024 + ro);
-      gx_ld(qh[hh], g + (8 + 2 * hh + h) * 1024 + ro);
+      qa[hh] = ld16(g + (4 * hh + h) * 1024 + ro);
+      qb[hh] = ld16(g + (4 * hh + 2 + h) * 1024 + ro);
+      qh[hh] = ld16(g + (8 + 2 * hh + h) * 1024 + ro);
     }
   }
   __device__ __forceinline__ static uint32_t codes(uint32_t ql, uint32_t qh, int k) {
@@ -286,7 +281,7 @@ template <class P> struct GxW<Q6_K, P> {
   }
   __device__ __forceinline__ h8 frag(const S& s, int u, int b, int h, h8& rest) const {
     const int hh = u >> 2, k = u & 3;
-    const P &c = k & 1 ? qb[hh] : qa[hh], &t = qh[hh];
+    const uint4 &c = k & 1 ? qb[hh] : qa[hh], &t = qh[hh];
     const uint32_t x = codes(first(c, b), first(t, b), k), y = codes(second(c, b), second(t, b), k);
     const h8 v = as_h8(x & 0x003F003Fu, (x >> 8) & 0x003F003Fu, y & 0x003F003Fu, (y >> 8) & 0x003F003Fu) -
                  splat8(32.f / 16777216.f);
@@ -300,7 +295,7 @@ template <class P> struct GxW<Q6_K, P> {
 };
 
 // Q8_0: codes of block u in chunks 2u + h, scales in chunk 16.
-template <class P> struct GxW<Q8_0, P> {
+template <> struct GxW<Q8_0> {
   static constexpr int GB = 64 * 272;
   struct S {
     uint4 s;
@@ -310,15 +305,15 @@ template <class P> struct GxW<Q8_0, P> {
     }
   };
   uint4 sc, scn;
-  P q[8];
+  uint4 q[8];
   __device__ __forceinline__ void load_head(const uint8_t* g, int row, int, int) { scn = ld16(g + 16 * 1024 + 16 * row); }
   __device__ __forceinline__ void next_head() { sc = scn; }
   __device__ __forceinline__ void load_body(const uint8_t* g, int ro, int h, int j) {
-    gx_ld(q[2 * j], g + (4 * j + h) * 1024 + ro);
-    gx_ld(q[2 * j + 1], g + (4 * j + 2 + h) * 1024 + ro);
+    q[2 * j] = ld16(g + (4 * j + h) * 1024 + ro);
+    q[2 * j + 1] = ld16(g + (4 * j + 2 + h) * 1024 + ro);
   }
   __device__ __forceinline__ h8 frag(const S&, int u, int b, int) const {
-    const P& c = q[u];
+    const uint4& c = q[u];
     const uint32_t x = first(c, b) ^ 0x80808080u, y = (second(c, b)) ^ 0x80808080u;
     return gx_ints(x & 0x00FF00FFu, (x >> 8) & 0x00FF00FFu, y & 0x00FF00FFu, (y >> 8) & 0x00FF00FFu, 128.f);
   }
