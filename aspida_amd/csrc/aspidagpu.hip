@@ -285,8 +285,9 @@ struct MvWorkspace {
 // the wave-per-column kernel (kq_mmw.hip), where the kind has one.
 // The pick is the many-vector kernel (kq_gemm.hip) where gemm_takes says so:
 // every kind above 64 vectors, and most batches above 4 to 16 on all but the
-// smallest matrices.  Below its line, for Q4_K and Q6_K (measured on MI355X at 4096x4096 and
-// 14336x4096, `small_batch` of bench.py):
+// smallest matrices.  Below its line the vector kernel, 8 vectors a launch, and
+// for Q4_K and Q6_K (measured on MI355X at 4096x4096 and 14336x4096,
+// `small_batch` of bench.py):
 //   up to 4 vectors: the batch-1 kernel on 4 vectors where its batch-1
 //     plan is 16-row workgroups (and Q6_K at 2 vectors), else one pass;
 //   5-16 vectors: one pass;
@@ -547,8 +548,7 @@ extern "C" void aspida_gpu_matmul(const void* w, long wbytes, int kind, int in_d
     return;
   }
   Ctx& c = ctx();
-  // Packed HBM mirror (shared with aspida_gpu_matvec): the multi-vector VALU
-  // kernel up to 8 vectors at a time, MFMA for larger Q4_K / Q6_K batches.
+  // Packed HBM mirror (shared with aspida_gpu_matvec), every kind by mm_route.
   std::shared_lock<std::shared_mutex> rd(g_wmu, std::defer_lock);
   WReq req = packed_req(w, kind, in_dim, out_dim);
   int rc = acquire(rd, &req, 1);

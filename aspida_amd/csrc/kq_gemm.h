@@ -345,14 +345,16 @@ __device__ __forceinline__ void gx_split(const float* x, int t, F&& frag, G&& su
 #pragma unroll
   for (int o = 1; o < 32; o <<= 1) a = fmaxf(a, __shfl_xor(a, o, 64));
   // S = 2^(14 - e) with a < 2^e, at most 2^116; 1 for a column of zeros.  Beside
-  // an Inf 2^-114, at which no finite element becomes one too.
+  // an Inf 2^-114, at which no finite element becomes one too: Q3_K and Q8_0,
+  // whose weight is one factor, then give the weight's sign times Inf.  The others
+  // give NaN (Q6_K's rest is mostly 0, a sum's second plane Inf - Inf).
   int e = 0;
   const bool inf = __builtin_isinf(a);
   if (a > 0.f && !inf) (void)frexpf(a, &e);
   const int ex = inf ? -114 : a > 0.f ? min(14 - e, 116) : 0;
   const float S = ldexpf(1.f, ex);
   if (t == 0) *reinterpret_cast<float*>(inv) = ldexpf(1.f, -ex);
-  // What hi leaves, at most 8; the clamp takes Inf - Inf, so that an Inf stays one.
+  // What hi leaves, at most 8; the clamp takes Inf - Inf.
   auto rest = [](float v, _Float16 hi) { return (_Float16)__builtin_amdgcn_fmed3f(v - (float)hi, -32.f, 32.f); };
   x0.x *= S; x0.y *= S; x0.z *= S; x0.w *= S;
   x1.x *= S; x1.y *= S; x1.z *= S; x1.w *= S;
@@ -577,7 +579,8 @@ __device__ __forceinline__ void gx_columns(const uint8_t* W, int row0, int s0, i
             for (int i = 0; i < 16; ++i) th[v][i] = __builtin_fmaf(x[i], d, th[v][i]);
           }
           // Holds the next pair's LDS reads back: without it the compiler
-          // spills 33 registers at NV = 2.
+          // spills 37 registers at NV = 2 in the products and up to 46 in the
+          // experts, with it 8 and up to 17.
           __builtin_amdgcn_sched_barrier(0);
         } else {
 #pragma unroll

@@ -9,11 +9,11 @@
 //                 with the columns split, the last workgroup adds the sums
 //
 // Bound by the matrix cores and the vector instructions around them: Q4_K
-// 28672x4096 x 512 takes 251 us, 0.96 PFLOP/s of f16 MFMA (hi and lo; a plain
-// f16 library product of the same MFMA work reaches 1.05), where eight launches
-// of the 64-vector kernel took 546; Q6_K 5001x3584 x 333 51 us (457 on the
-// one-pass kernel, 32 vectors a launch), Q6_K 4096x14336 x 64 40 us (115), Q5_K
-// 14336x4096 x 16 21 us (109 on the vector kernel, 8 vectors a launch).
+// 28672x4096 x 512 takes 251 to 256 us, 0.95 PFLOP/s of f16 MFMA (hi and lo; a
+// plain f16 library product of 8192^3 reaches 1.12), where eight launches of the
+// 64-vector kernel took 546; Q6_K 5001x3584 x 333 49 us (457 on the one-pass
+// kernel, 32 vectors a launch), Q6_K 4096x14336 x 64 38 us (115), Q5_K
+// 14336x4096 x 16 20 us (109 on the vector kernel, 8 vectors a launch).
 // Measured and not kept: decoding a stage ahead into LDS for two waves (tile
 // 128 x 64 shared, 292 against 260 us) or four (128 x 128, 331): the waits at
 // its barriers cost more than the instructions saved; 64 rows x 32 vectors a

@@ -27,10 +27,10 @@
 // Bound by the matrix cores and the vector instructions around them (kq_gemm.h)
 // from about 100 tokens, by the weights' latency below.  The Qwen3-MoE layer
 // (2048x768, 128 experts and a shared one, top 8, Q4_K / Q6_K, router included):
-// 1024 tokens 429 us (889 on 16x16x16 products of 64-job tiles), 512 283 (474),
-// 256 200 (352), 128 184 (265), 64 166 (216); Q5_K / Q6_K 256 tokens 205 (1468
-// on the vector ALUs).  At 1024: router 30, prep 12, gate/up 236, h split 14,
-// down 155, combine 22.
+// 1024 tokens 419 us (890 on 16x16x16 products of 64-job tiles), 512 265 (465),
+// 256 179 (353), 128 162 (266), 64 153 (212 on two-job chunks); Q5_K / Q6_K 256
+// tokens 190 (1457 on the vector ALUs).  At 1024 under the profiler, shortest of
+// 20 launches: router 28, prep 11, gate/up 211, h split 13, down 139, combine 21.
 #include <math.h>
 
 #include <algorithm>

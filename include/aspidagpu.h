@@ -413,8 +413,8 @@ int aspida_kq_set_mv_engine(int engine);
 /* Engine of the packed small-batch product (batch > 1 in
  * aspida_kq_matmul_packed_dev and aspida_gpu_matmul): 0 = the built-in choice
  * (the many-vector kernel wherever it measured ahead: every kind above 64
- * vectors, most matrices above 4 to 16; below that line, Q4_K and Q6_K: up to 4 vectors on the batch-1 matrix-core kernel where
- * the batch-1 plan is 16-row workgroups, else the one-pass kernel -- Q6_K
+ * vectors, most matrices above 4 to 16; below that line, Q4_K and Q6_K: up to 4
+ * vectors on the batch-1 matrix-core kernel where the batch-1 plan is 16-row workgroups, else the one-pass kernel -- Q6_K
  * keeps the batch-1 kernel at 2 vectors -- then the one-pass kernel up to
  * 16 vectors (on matrices of at least 8192 64-row-by-256-column blocks,
  * such as output heads, the 16-vector matrix-core kernel instead, Q6_K from
