@@ -197,7 +197,9 @@ bool gemm_takes(int kind, int in_dim, int out_dim, int batch) {
       // 20.1, but 2048^2 15.8 / 14.1.
       if (batch > 32) return nsb >= 16;
       // 17..32: 14336x4096 20.5 / 25.3, 4096x8192 17.6 / 19.2, 8192x4096 16.0 /
-      // 16.7, 4096^2 13.2 / 14.0, 1024x4096 12.5 / 12.6, but 2048^2 10.8 / 10.4.
+      // 16.7, 4096^2 13.2 / 14.0, 1024x4096 12.5 / 12.6, but 2048^2 10.8 / 10.4;
+      // on shorter rows many tiles only (18944x3584 22.1 / 33.9, 49152x2048 26.4 /
+      // 34.2 at 17).
       if (batch > 16) return nsb >= 16 || units >= 3584;
       // Up to 16 only against 16-row blocks: 8192x4096 15.3 / 18.9 at 12,
       // 8192^2 21.3 / 29.2 at 8, 4096x14336 23.7 / 27.0 at 6, but 14336x4096
